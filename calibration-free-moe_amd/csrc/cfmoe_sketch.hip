@@ -21,7 +21,7 @@
 // blocks 128 body + ((b / 2) 128 + c) 32 + (b % 2) 16. The FP16 statistics
 // go to the physical [E, blocks, 2, 2 I] layout (scale plane, residual plane).
 //
-// The sums behind mean|v|, the scale and the residual are wave trees, not
+// The sums behind mean|v|, the scale and the residual are xor trees, not
 // torch's reduction order: the threshold test can differ from a torch build
 // only for |v| within an FP32 rounding of 0.7 mean|v|, and the FP16
 // statistics only by a rounding.
@@ -29,6 +29,8 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "cfmoe_reader.h"
 
@@ -45,92 +47,219 @@ constexpr float kRotationScale = 0.08838834764831845f;  // fp32(1 / sqrt(128))
 struct SketchArgs {
   const uint16_t *weights;  // [E, 2 I, H] bf16
   const int8_t *signs;      // [H] +-1, or NULL (unrotated blocks)
-  uint8_t *codes;           // [E, storage], padding bytes already 121
+  uint8_t *codes;           // [E, storage]
   __half *stats;            // physical [E, blocks, 2, 2 I]
   long storage;
   int rows, width, hidden, blocks, groups, stride, body;
+  int tiles;  // kTileColumns-byte columns of a coordinate's code run
 };
 
-__device__ __forceinline__ float bf16_value(uint16_t h) {
-  return __uint_as_float(static_cast<uint32_t>(h) << 16);
+// Loads and stores at the element's own alignment: callers' tensors may be
+// views at any element offset (one wide access each all the same).
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x4 row_words __attribute__((aligned(2)));
+typedef u32x2 sign_words __attribute__((aligned(1)));
+typedef uint32_t code_word __attribute__((aligned(1)));
+
+// Eight lanes of a wave share one row's block: lane i of the eight holds the
+// coordinates 8 y .. 8 y + 7 and 64 + 8 y .. 64 + 8 y + 7 with y = (i & 3) ^
+// (i & 4 ? 7 : 0), so that the lanes whose y differ in bit 0, 1 or 2 are i ^ 1,
+// i ^ 2 and i ^ 7: one DPP move each (two quad permutes, the half-row mirror).
+constexpr int kRowLanes = 8;
+constexpr int kLaneValues = 16;
+constexpr int kExchange[3] = {0xb1, 0x4e, 0x141};
+
+template <int kControl>
+__device__ __forceinline__ float partner(float v) {
+  // (bound_ctrl set: the move folds into the add that uses it)
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kControl, 0xf, 0xf, true));
 }
 
-// Sum over the wave in a fixed xor-butterfly order; every lane gets it.
-__device__ __forceinline__ float wave_total(float v) {
+// Sum of a block's 128 values, every lane of the eight gets it: coordinates c
+// and c + 64 first, then the xor tree over c's bits 0 .. 5 (the order of a
+// 64-lane wave tree over lanes c that each hold c and c + 64).
+__device__ __forceinline__ float block_total(const float (&v)[kLaneValues]) {
+  float t[8];
 #pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v = v + __shfl_xor(v, m);
-  return v;
+  for (int i = 0; i < 8; ++i) t[i] = v[i] + v[8 + i];
+  float sum = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+  sum = sum + partner<kExchange[0]>(sum);
+  sum = sum + partner<kExchange[1]>(sum);
+  return sum + partner<kExchange[2]>(sum);
 }
 
-// Workgroup = one wave per (expert e, block b, plane, group g of five
-// channels); lane l handles coordinates l and l + 64 of the block.
-__global__ __launch_bounds__(64) void build_sketch_kernel(SketchArgs a) {
-  const int lane = threadIdx.x;
-  long item = blockIdx.x;
-  const int g = static_cast<int>(item % a.groups);
-  item /= a.groups;
-  const int plane = static_cast<int>(item % 2);
-  item /= 2;
-  const int b = static_cast<int>(item % a.blocks);
-  const int e = static_cast<int>(item / a.blocks);
+constexpr int kTileColumns = 64;              // code bytes of a coordinate per workgroup
+constexpr int kTileThreads = kTileColumns * kRowLanes;
+constexpr int kTileStride = kTileColumns + 4;  // LDS bytes per coordinate (bank spread)
+constexpr int kTileChannels = 5 * kTileColumns / 2;
+
+// Workgroup = (expert e, 64 code byte columns, block b), eight lanes per
+// column: the column's five rows (channels 5 g .. 5 g + 4 of one plane) are
+// loaded together, each lane keeps the codes of its 16 coordinates in
+// registers, and the tile's bytes and statistics leave through LDS as whole
+// words. Every byte of the block's code rows is written (padding columns, and
+// the missing half of an odd block count's last tail rows, hold 121).
+//
+// Bound by the vector unit (about 470 instructions per eight row blocks: 176
+// of them the butterflies): a 128-expert layer of 1536 x 2048 rows takes 262
+// us, 3.4 TB/s of its 898 MB, where the instructions alone take about 250. A
+// wave per column with two coordinates per lane took 990 us, in single-byte
+// stores `body` bytes apart, LDS exchanges for every butterfly and three
+// 64-lane trees per row. The tile is 64 bytes because a coordinate's run then
+// leaves as one 64-byte piece.
+template <bool kRotate>
+__global__ __launch_bounds__(kTileThreads) void build_sketch_kernel(SketchArgs a) {
+  __shared__ __align__(16) uint8_t tile[128 * kTileStride];
+  __shared__ __half tile_stats[2][2][kTileChannels];  // [plane][scale, residual][channel]
+  const int tid = threadIdx.x;
+  int item = blockIdx.x;
+  const int b = item % a.blocks;
+  item /= a.blocks;
+  const int column0 = item % a.tiles * kTileColumns;
+  const int e = item / a.tiles;
+  const int local = tid / kRowLanes, j = column0 + local;
+  const int plane = j & 1, g = j >> 1;
+  const int i8 = tid % kRowLanes, y = (i8 & 3) ^ (i8 & 4 ? 7 : 0);
   const int base = b * 128;
-  float sign0 = 1.0f, sign1 = 1.0f;
-  if (a.signs) {
-    sign0 = static_cast<float>(a.signs[base + lane]);
-    sign1 = static_cast<float>(a.signs[base + 64 + lane]);
-  }
-  int code0 = 0, code1 = 0, power = 1;
-  for (int d = 0; d < 5; ++d, power *= 3) {
-    const int channel = 5 * g + d;
-    if (channel >= a.width) {  // past the width: zero trit, digit 1
-      code0 += power;
-      code1 += power;
-      continue;
-    }
-    const int row = plane * a.width + channel;
-    const uint16_t *source = a.weights + (static_cast<long>(e) * a.rows + row) * a.hidden + base;
-    float v0 = bf16_value(source[lane]), v1 = bf16_value(source[64 + lane]);
-    if (a.signs) {
-      v0 = v0 * sign0;
-      v1 = v1 * sign1;
+  const bool live = g < a.groups;
+
+  u32x4 words[5][2];
+  const uint16_t *rows = a.weights + (static_cast<long>(e) * a.rows + plane * a.width) * a.hidden + base + 8 * y;
 #pragma unroll
-      for (int stage = 0; stage < 6; ++stage) {
-        const int bit = 1 << stage;
-        const float p0 = __shfl_xor(v0, bit), p1 = __shfl_xor(v1, bit);
-        v0 = (lane & bit) ? p0 - v0 : v0 + p0;
-        v1 = (lane & bit) ? p1 - v1 : v1 + p1;
-      }
-      const float sum = v0 + v1, difference = v0 - v1;
-      v0 = sum * kRotationScale;
-      v1 = difference * kRotationScale;
-    }
-    const float m0 = fabsf(v0), m1 = fabsf(v1);
-    const float threshold = 0.7f * (wave_total(m0 + m1) / 128.0f);
-    const bool keep0 = m0 > threshold, keep1 = m1 > threshold;
-    const int kept = __popcll(__ballot(keep0)) + __popcll(__ballot(keep1));
-    const float kept_sum = wave_total((keep0 ? m0 : 0.0f) + (keep1 ? m1 : 0.0f));
-    const float scale = kept_sum / static_cast<float>(kept > 1 ? kept : 1);
-    const float t0 = keep0 ? (v0 > 0.0f ? 1.0f : -1.0f) : 0.0f;
-    const float t1 = keep1 ? (v1 > 0.0f ? 1.0f : -1.0f) : 0.0f;
-    const float r0 = v0 - t0 * scale, r1 = v1 - t1 * scale;
-    const float residual = wave_total(r0 * r0 + r1 * r1) / 128.0f;
-    if (lane == 0) {
-      __half *stats = a.stats + (static_cast<long>(e) * a.blocks + b) * 2 * a.rows + row;
-      stats[0] = __float2half_rn(scale);
-      stats[a.rows] = __float2half_rn(residual);
-    }
-    code0 += (static_cast<int>(t0) + 1) * power;
-    code1 += (static_cast<int>(t1) + 1) * power;
+  for (int d = 0; d < 5; ++d) {
+    // (a channel past the width reads the last one; its trits stay zero)
+    const long row = static_cast<long>(min(5 * g + d, a.width - 1)) * a.hidden;
+    words[d][0] = *reinterpret_cast<const row_words *>(rows + row);
+    words[d][1] = *reinterpret_cast<const row_words *>(rows + row + 64);
   }
-  const int j = 2 * g + plane;
+  float sign[kLaneValues];
+  if (kRotate) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const u32x2 s = *reinterpret_cast<const sign_words *>(a.signs + base + 64 * h + 8 * y);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        sign[8 * h + i] = static_cast<float>(static_cast<int8_t>((i < 4 ? s.x : s.y) >> (8 * (i & 3))));
+    }
+  }
+  // the upper half of a cross-lane butterfly subtracts: its own value negated
+  uint32_t negate[3];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) negate[s] = (y >> s) & 1 ? 0x80000000u : 0u;
+
+  float code[kLaneValues];  // 121 + sum_d t_d 3^d
+#pragma unroll
+  for (int i = 0; i < kLaneValues; ++i) code[i] = 121.0f;
+  float power = 1.0f;
+#pragma unroll
+  for (int d = 0; d < 5; ++d, power *= 3.0f) {
+    float v[kLaneValues];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[8 * h + 2 * i] = __uint_as_float(words[d][h][i] << 16);
+        v[8 * h + 2 * i + 1] = __uint_as_float(words[d][h][i] & 0xffff0000u);
+      }
+    if (kRotate) {
+#pragma unroll
+      for (int i = 0; i < kLaneValues; ++i) v[i] = v[i] * sign[i];
+      auto within = [&](int width) {  // coordinates of the lane's own registers
+#pragma unroll
+        for (int i = 0; i < kLaneValues; ++i) {
+          if (i & width) continue;
+          const float low = v[i], high = v[i + width];
+          v[i] = low + high;
+          v[i + width] = low - high;
+        }
+      };
+      auto across = [&](auto stage) {  // the partner lane's
+        constexpr int kStage = decltype(stage)::value;
+#pragma unroll
+        for (int i = 0; i < kLaneValues; ++i)
+          v[i] = __uint_as_float(__float_as_uint(v[i]) ^ negate[kStage]) + partner<kExchange[kStage]>(v[i]);
+      };
+      within(1);
+      within(2);
+      within(4);
+      across(std::integral_constant<int, 0>());
+      across(std::integral_constant<int, 1>());
+      across(std::integral_constant<int, 2>());
+      within(8);  // coordinates 64 apart
+#pragma unroll
+      for (int i = 0; i < kLaneValues; ++i) v[i] = v[i] * kRotationScale;
+    }
+    float m[kLaneValues];
+#pragma unroll
+    for (int i = 0; i < kLaneValues; ++i) m[i] = fabsf(v[i]);
+    const float threshold = 0.7f * (block_total(m) / 128.0f);
+    int kept = 0;
+    float kept_m[kLaneValues];
+#pragma unroll
+    for (int i = 0; i < kLaneValues; ++i) {
+      kept += m[i] > threshold;
+      kept_m[i] = m[i] > threshold ? m[i] : 0.0f;
+    }
+    kept += __builtin_amdgcn_mov_dpp(kept, kExchange[0], 0xf, 0xf, false);
+    kept += __builtin_amdgcn_mov_dpp(kept, kExchange[1], 0xf, 0xf, false);
+    kept += __builtin_amdgcn_mov_dpp(kept, kExchange[2], 0xf, 0xf, false);
+    const float scale = block_total(kept_m) / static_cast<float>(max(kept, 1));
+    // (v - t scale)^2 = (|v| - [kept] scale)^2
+    float square[kLaneValues];
+#pragma unroll
+    for (int i = 0; i < kLaneValues; ++i) {
+      const float r = m[i] - (m[i] > threshold ? scale : 0.0f);
+      square[i] = r * r;
+    }
+    const float residual = block_total(square) / 128.0f;
+    const bool inside = live && 5 * g + d < a.width;
+    const float trit = inside ? power : 0.0f;
+#pragma unroll
+    for (int i = 0; i < kLaneValues; ++i)
+      code[i] = code[i] + (m[i] > threshold ? copysignf(trit, v[i]) : 0.0f);
+    if (i8 == 0) {
+      const int channel = 5 * (local >> 1) + d;
+      tile_stats[plane][0][channel] = __float2half_rn(scale);
+      tile_stats[plane][1][channel] = __float2half_rn(residual);
+    }
+    // (each row's codes are done before the next row begins: left to the end,
+    // the five rows' kept masks would not fit the scalar registers)
+#pragma unroll
+    for (int i = 0; i < kLaneValues; ++i) asm volatile("" : "+v"(code[i]));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int i = 0; i < kLaneValues; ++i)
+    tile[(64 * (i >> 3) + 8 * y + (i & 7)) * kTileStride + local] = static_cast<uint8_t>(static_cast<int>(code[i]));
+  __syncthreads();
+
+  // the tile's code words: bytes [0, body) of a coordinate in the block's
+  // body, [body, stride) in its half of the block pair's tail row
   uint8_t *codes = a.codes + static_cast<long>(e) * a.storage;
-  auto offset = [&](int c) -> long {
-    if (j < a.body) return static_cast<long>(base + c) * a.body + j;
-    return static_cast<long>(a.blocks) * 128 * a.body + ((b / 2) * 128 + c) * 32 + (b % 2) * 16 +
-           (j - a.body);
-  };
-  codes[offset(lane)] = static_cast<uint8_t>(code0);
-  codes[offset(lane + 64)] = static_cast<uint8_t>(code1);
+  const long tails = static_cast<long>(a.blocks) * 128 * a.body;
+  constexpr int kRunWords = kTileColumns / 4;
+#pragma unroll
+  for (int n = 0; n < 128 * kRunWords / kTileThreads; ++n) {
+    const int at = tid + n * kTileThreads;
+    const int c = at / kRunWords, byte = 4 * (at % kRunWords), column = column0 + byte;
+    if (column >= a.stride) continue;
+    const uint32_t word = *reinterpret_cast<const uint32_t *>(&tile[c * kTileStride + byte]);
+    if (column < a.body) {
+      *reinterpret_cast<code_word *>(codes + static_cast<long>(base + c) * a.body + column) = word;
+    } else {
+      const long row = tails + ((b / 2) * 128 + c) * 32 + (column - a.body);
+      *reinterpret_cast<code_word *>(codes + row + (b % 2) * 16) = word;
+      // (an odd block count's last tail rows have no second block)
+      if (b % 2 == 0 && b + 1 == a.blocks) *reinterpret_cast<code_word *>(codes + row + 16) = 0x79797979u;
+    }
+  }
+  __half *stats = a.stats + (static_cast<long>(e) * a.blocks + b) * 2 * a.rows;
+  for (int at = tid; at < 4 * kTileChannels; at += kTileThreads) {
+    const int p = at / (2 * kTileChannels), which = at / kTileChannels % 2, within = at % kTileChannels;
+    const int channel = 5 * (column0 / 2) + within;
+    if (channel < a.width) stats[which * a.rows + p * a.width + channel] = tile_stats[p][which][within];
+  }
 }
 
 }  // namespace
@@ -160,9 +289,14 @@ CFMOE_API int cfmoe_build_sketch(int32_t experts, int32_t width, int32_t hidden,
   a.body = a.stride - a.stride % 32;
   const long tail = a.stride % 32 ? static_cast<long>((a.blocks + 1) / 2) * 128 * 32 : 0;
   a.storage = static_cast<long>(a.blocks) * 128 * a.body + tail;
-  const long items = static_cast<long>(experts) * a.blocks * 2 * a.groups;
-  hipLaunchKernelGGL(build_sketch_kernel, dim3(static_cast<unsigned>(items)), dim3(64), 0, stream,
-                     a);
+  a.tiles = (a.stride + kTileColumns - 1) / kTileColumns;
+  const long items = static_cast<long>(experts) * a.tiles * a.blocks;
+  if (items > 0x7fffffffL) return fail(CFMOE_EINVAL, "sketch has too many blocks for one launch");
+  const dim3 grid(static_cast<unsigned>(items));
+  if (a.signs)
+    hipLaunchKernelGGL(build_sketch_kernel<true>, grid, dim3(kTileThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL(build_sketch_kernel<false>, grid, dim3(kTileThreads), 0, stream, a);
   return check_launch("build_sketch");
 }
 

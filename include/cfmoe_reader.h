@@ -205,9 +205,8 @@ CFMOE_API int cfmoe_unpack_trit_planes(const cfmoe_dims *dims, const uint32_t *t
  * `signs` [hidden] +-1 int8 or none when NULL, TWN ternarisation per
  * 128-coordinate block, five trits per byte, body/tail byte layout) in one
  * launch instead of its per-expert torch loop. `codes` [experts,
- * sketch_storage_bytes] must hold 121 (five zero trits) in every byte before
- * the call (the kernel writes only the bytes that carry channels);
- * `statistics` is fp16 in the physical [experts, hidden / 128, 2, 2 width]
+ * sketch_storage_bytes] is written in every byte (121, five zero trits, in
+ * those that carry no channel); `statistics` is fp16 in the physical [experts, hidden / 128, 2, 2 width]
  * layout (scale plane, residual plane). */
 CFMOE_API int cfmoe_build_sketch(int32_t experts, int32_t width, int32_t hidden,
                                  const void *gate_up, const int8_t *signs, uint8_t *codes,

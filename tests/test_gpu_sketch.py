@@ -78,3 +78,37 @@ def test_default_build_on_the_device_is_the_torch_construction():
     torch.cuda.synchronize()
     assert torch.equal(got_codes.cpu(), want_codes)
     torch.testing.assert_close(got_stats.cpu(), want_stats, atol=1e-4, rtol=1e-3)
+
+
+@pytest.mark.parametrize(
+    "experts,width,hidden,offset",
+    # one tile of code columns holds 160 channels: a part of one, one, one and
+    # a channel, with rows and signs that start at odd elements; one block (an
+    # odd count's tail), and the largest widths
+    [(2, 33, 128, 1), (2, 160, 384, 3), (1, 161, 640, 5), (1, 2048, 256, 0), (1, 80, 4096, 7)],
+)
+def test_device_sketch_tiles_and_offsets(experts, width, hidden, offset):
+    """Tile edges and views at any element offset, on memory that holds no
+    code bytes of its own beforehand (0xff is no code)."""
+    generator = torch.Generator().manual_seed(width + offset)
+    flat = (torch.randn(offset + experts * 2 * width * hidden, generator=generator) * 0.02).bfloat16()
+    weights = flat[offset:].view(experts, 2 * width, hidden)
+    signs = block_hadamard_signs(hidden, "cpu")
+    want_codes, want_stats = build_sketch(weights, signs)
+    stale = torch.full_like(want_codes, 0xFF).to(DEVICE)
+    del stale  # (the next allocation of this size may take its memory)
+    device_signs = torch.cat([torch.zeros(offset, dtype=torch.int8), signs]).to(DEVICE)[offset:]
+    got_codes, got_stats = build_sketch(
+        flat.to(DEVICE)[offset:].view(experts, 2 * width, hidden), device_signs, device_kernel=True
+    )
+    torch.cuda.synchronize()
+    value = rotate_blocks(weights, signs).reshape(experts, 2 * width, hidden // 128, 128).double()
+    threshold = 0.7 * value.abs().mean(-1, keepdim=True)
+    near = (value.abs() - threshold).abs() <= 2e-5 * threshold
+    differ = (unpack_sketch(got_codes.cpu(), 2 * width, hidden)
+              != unpack_sketch(want_codes, 2 * width, hidden)).reshape(near.shape)
+    assert not (differ & ~near).any()
+    assert int((got_codes.cpu() != want_codes).sum()) <= int(differ.sum())
+    clean = ~differ.any(-1)
+    torch.testing.assert_close(got_stats.cpu().float()[clean], want_stats.float()[clean],
+                               rtol=1e-3, atol=1e-4)
