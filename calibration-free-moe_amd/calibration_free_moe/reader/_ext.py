@@ -23,6 +23,7 @@ ACCOUNT = 16
 IDS_INT64 = 32
 WEIGHTS_BF16 = 64
 INPUT_PREPARED = 128
+CHARGE_KEPT = 256
 
 EINVAL = 1
 EHIP = 2

@@ -633,14 +633,12 @@ class ProgressiveReader:
         )
         self._workspace_c = workspace.pointers(self.read_work)
         self._workspace_c.next_ids = _pointer(self.candidate_ids[1])
-        # per-token read charges of per-token and of grouped calls; thresholded
-        # readers add theirs from the selection (the device still adds its
-        # per-tile and union terms)
+        # per-token read charges of per-token and of grouped calls
         charges = (ctypes.c_double * 18)
         self._charges = {
             grouped: charges(*(
                 self._fixed_charges(grouped, grouped) if selection_threshold is None
-                else (0.0,) * 18))
+                else self._threshold_charges(grouped)))
             for grouped in (False, True)
         }
         _ext.library()
@@ -696,6 +694,25 @@ class ProgressiveReader:
             )
         )
 
+    def _threshold_charges(self, grouped: bool) -> tuple[float, ...]:
+        """The part of a thresholded token's statistics that no selection changes.
+
+        The kept count varies per token (progressive.py:2189-2225): its rows'
+        bytes (slots 0, 6, 12, 13), the encoder rows it leaves out (3, 7) and
+        slot 19 are added by the selection on the device (CHARGE_KEPT), the
+        per-tile screen terms and grouped union rows as in every call. Slots 4
+        and 9 also price the threshold itself (4 bytes, a 32-byte sector).
+        """
+        p = self.plan
+        charges = list(self._fixed_charges(grouped, grouped))
+        for slot in (0, 6, 12, 13):
+            charges[slot] = 0.0
+        for slot in (3, 7):
+            charges[slot] = 2.0 * self.rank * (p.candidate_count + p.hidden_size)
+        charges[4] += 4.0
+        charges[9] += 32.0
+        return tuple(charges)
+
     def _flags(self, ids: Tensor, weights: Tensor, input_prepared: bool) -> int:
         flags = 0
         if self.selection_score == "point":
@@ -705,7 +722,7 @@ class ProgressiveReader:
         if self.recovery_geometry is not None:
             flags |= _ext.GEOMETRY
         if self.selection_threshold is not None:
-            flags |= _ext.THRESHOLD
+            flags |= _ext.THRESHOLD | _ext.CHARGE_KEPT
         flags |= _ext.ACCOUNT
         if ids.dtype == torch.int64:
             flags |= _ext.IDS_INT64
@@ -894,8 +911,6 @@ class ProgressiveReader:
                 self._stream(),
             )
         )
-        if self.selection_threshold is not None:
-            self._charge_thresholded(tokens, padding)
         return out
 
     def launch_stage(
@@ -933,56 +948,6 @@ class ProgressiveReader:
                 self._stream(),
             )
         )
-
-    def _charge_thresholded(self, tokens: int, padding: Tensor | None) -> None:
-        """Selection-dependent read statistics of a thresholded call.
-
-        Enqueued torch ops on the current stream (no host sync): the kept count
-        varies per token, so charges follow progressive.py:2189-2225 with the
-        per-token selected counts. The device adds the per-tile screen terms
-        (slots 11, 15) and, in grouped calls, the union rows (slot 12).
-        """
-        p = self.plan
-        h, i, k, n, rank = (
-            p.hidden_size, p.expert_width, p.top_k, p.candidate_count, self.rank
-        )
-        active = (
-            torch.ones(tokens, dtype=torch.float64, device=self.read_work.device)
-            if padding is None
-            else (~padding).to(torch.float64)
-        )
-        selected = self.selected[:tokens].sum(1).to(torch.float64) * active
-        completed = self.completed[:tokens].sum(1).to(torch.float64) * active
-        count = active.sum()
-        kept = selected.sum()
-        done = completed.sum()
-        geometry = self.recovery_geometry is not None
-        residual = self.selection_score != "point"
-        candidates = count * n
-        native = 2 * (2 * done * h + kept * h)
-        recovery = 2 * rank * (candidates - kept + count * h)
-        selection = (12 if geometry else 4) * candidates + 4 * count
-        physical_selection = (12 if geometry else 4) * candidates + 32 * count
-        sketch = count * p.sketch_read_bytes(residual, sectors=False)
-        physical_sketch = count * p.sketch_read_bytes(residual)
-        work = self.read_work
-        work[0] += native
-        work[1] += count * p.native_read_bytes()
-        work[3] += recovery
-        work[4] += selection
-        work[5] += sketch
-        work[6] += native
-        work[7] += recovery
-        work[9] += physical_selection
-        work[10] += count * h
-        if tokens >= self.grouped_tokens:
-            work[16] += count
-        else:
-            work[12] += 2 * 2 * h * done
-        work[13] += 2 * h * kept
-        work[14] += 2 * rank * candidates
-        work[17] += physical_sketch
-        work[19] += count
 
     def report(self) -> dict[str, float | None]:
         """Accumulated read statistics and work counters (progressive.py:3517-3803).

@@ -1778,6 +1778,12 @@ struct SelectArgs {
   int32_t *down_tile_starts;
   int N, F, I, K;
   int thresholded;
+  // read statistics of the kept count (kCharge), or NULL: rows of
+  // hidden size H, encoder rows of rank R; `row_charge` is slot 12's bytes per
+  // kept channel (0 in grouped calls, whose union rows the exact launch counts)
+  double *read_work;
+  const uint8_t *padding;
+  int H, R, row_charge;
 };
 
 constexpr int kSelectThreads = 1024;
@@ -1865,7 +1871,7 @@ __device__ __forceinline__ int select_wide(const int *histogram, int *totals, in
 // outputs: kept ids, selected flags, completed flags (zeros, or with
 // `completed_kept` the selected flags, which the exact rows of a launch that
 // also runs them set anyway), slot records and tile mask bits.
-template <int kKeys>  // keys per thread: N <= kKeys * kSelectThreads
+template <int kKeys, bool kCharge>  // keys per thread: N <= kKeys * kSelectThreads
 __device__ __forceinline__ void select_token(const SelectArgs &a, int t, bool write, bool completed_kept,
                                              uint32_t *kept_out, int *base_out) {
   __shared__ int wide[2][kSelectWideSlots];
@@ -2059,6 +2065,16 @@ __device__ __forceinline__ void select_token(const SelectArgs &a, int t, bool wr
   for (int p = kept_total + tid; p < a.F; p += kSelectThreads)
     a.next_ids[static_cast<long>(t) * a.F + p] = -1;
   if (tid == 0) slot_start[a.K] = min(kept_total, a.F);
+  // the kept count's read statistics (integers, exact in FP64 in any order),
+  // one slot per lane of wave 1 (a template argument: the test alone cost the
+  // batch-1 calls that never charge 0.3 us)
+  if (kCharge && wave == 1 && lane < 7 && is_active(a.padding, t)) {
+    const int kept_slots[7] = {0, 6, 13, 12, 3, 7, 19};
+    const int slot = kept_slots[lane];
+    const double bytes = lane < 2 ? 6.0 * a.H : lane == 2 ? 2.0 * a.H : lane == 3 ? a.row_charge : -2.0 * a.R;
+    const double charge = lane == 6 ? 1.0 : bytes * min(kept_total, a.F);
+    if (charge != 0.0) atomicAdd(a.read_work + slot, charge);
+  }
   __syncthreads();
   // wave 0: lane k writes slot k's count, start and tile starts (K <= 64)
   if (tid < kWave) {
@@ -2076,11 +2092,11 @@ __device__ __forceinline__ void select_token(const SelectArgs &a, int t, bool wr
   }
 }
 
-template <int kKeys>
+template <int kKeys, bool kCharge>
 __global__ __launch_bounds__(kSelectThreads) void select_kernel(SelectArgs a) {
   uint32_t kept;
   int base;
-  select_token<kKeys>(a, blockIdx.x, true, false, &kept, &base);
+  select_token<kKeys, kCharge>(a, blockIdx.x, true, false, &kept, &base);
 }
 
 // Full retention: every candidate is kept (progressive.py:2999-3004).
@@ -2932,7 +2948,7 @@ __global__ __launch_bounds__(64) void exact_kernel(ExactArgs a) {
 // before the selection. The host sizes item_waves so that the workgroups
 // (one per compute unit at 16 waves of this kernel's registers) run in one
 // round: the rows then come through as many compute units as that allows.
-template <int kKeys, int kParts>
+template <int kKeys, int kParts, bool kCharge>
 __global__ __launch_bounds__(kSelectThreads) void select_exact_kernel(SelectArgs s, ExactArgs a,
                                                                       int item_waves) {
   __shared__ int kept_end[kSelectThreads];
@@ -2946,7 +2962,7 @@ __global__ __launch_bounds__(kSelectThreads) void select_exact_kernel(SelectArgs
       __builtin_amdgcn_raw_buffer_load_b8(buffer_resource(a.padding_source, a.padding_bytes), t, 0, 0);
   uint32_t kept;
   int base;
-  select_token<kKeys>(s, t, writer, true, &kept, &base);
+  select_token<kKeys, kCharge>(s, t, writer, true, &kept, &base);
   if (writer) return;
   kept_end[tid] = base + __builtin_popcount(kept);
   kept_bits[tid] = kept;
@@ -3775,6 +3791,12 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   const bool masked = s.screened && grouped;
   sel.pair_tiles = workspace->pair_tiles;
   sel.tile_masks = masked ? workspace->tile_masks : nullptr;
+  const uint32_t charge_kept = CFMOE_ACCOUNT | CFMOE_CHARGE_KEPT;
+  sel.read_work = (flags & charge_kept) == charge_kept ? workspace->read_work : nullptr;
+  sel.padding = padding;
+  sel.H = s.H;
+  sel.R = s.R;
+  sel.row_charge = grouped ? 0 : 4 * s.H;
   // Up to kSelectExactTokens tokens a call that runs both stages runs select
   // and exact as one launch (select_exact_kernel, in the exact launch's place)
   // when its workgroups at 16 item waves each fit on the compute units at
@@ -3859,11 +3881,12 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
     }
 
     if ((stages & (1u << CFMOE_STAGE_SELECT)) && !fuse_select) {
-      if (s.N <= 8 * kSelectThreads)
-        hipLaunchKernelGGL(select_kernel<8>, dim3(tokens), dim3(kSelectThreads), 0, stream, sel);
-      else
-        hipLaunchKernelGGL(select_kernel<kSelectKeys>, dim3(tokens), dim3(kSelectThreads), 0,
-                           stream, sel);
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(tokens), dim3(kSelectThreads), 0, stream, sel);
+      };
+      const bool few = s.N <= 8 * kSelectThreads;
+      if (sel.read_work) launch(few ? select_kernel<8, true> : select_kernel<kSelectKeys, true>);
+      else launch(few ? select_kernel<8, false> : select_kernel<kSelectKeys, false>);
       if ((rc = check_launch("select"))) return rc;
     }
   } else if (stages & (1u << CFMOE_STAGE_SELECT)) {
@@ -3985,12 +4008,16 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
       const int item_waves =
           static_cast<int>(std::min<long>(kSelectWaves, std::max<long>(1, (items + groups - 1) / groups)));
       const dim3 grid(1 + (items + item_waves - 1) / item_waves, tokens);
-      if (s.N <= 8 * kSelectThreads)
-        hipLaunchKernelGGL((select_exact_kernel<8, kNarrowParts>), grid, dim3(kSelectThreads), 0, stream, sel, ex,
-                           item_waves);
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kSelectThreads), 0, stream, sel, ex, item_waves);
+      };
+      const bool few = s.N <= 8 * kSelectThreads;
+      if (sel.read_work)
+        launch(few ? select_exact_kernel<8, kNarrowParts, true>
+                   : select_exact_kernel<kSelectKeys, kNarrowParts, true>);
       else
-        hipLaunchKernelGGL((select_exact_kernel<kSelectKeys, kNarrowParts>), grid, dim3(kSelectThreads), 0, stream,
-                           sel, ex, item_waves);
+        launch(few ? select_exact_kernel<8, kNarrowParts, false>
+                   : select_exact_kernel<kSelectKeys, kNarrowParts, false>);
     } else if (hidden_parts(s.H) == kNarrowParts)
       hipLaunchKernelGGL(exact_kernel<kNarrowParts>, dim3(s.F + (encode_items + 1) / 2, tokens), dim3(kWave), 0,
                          stream, ex);

@@ -47,6 +47,10 @@ typedef struct ihipStream_t *cfmoe_stream;
 #define CFMOE_IDS_INT64 32u     /* router ids are int64 (else int32) */
 #define CFMOE_WEIGHTS_BF16 64u  /* router weights are bf16 (else fp32) */
 #define CFMOE_INPUT_PREPARED 128u /* cfmoe_prepare_input already rotated */
+#define CFMOE_CHARGE_KEPT 256u  /* with CFMOE_ACCOUNT: also add the read statistics that
+                                   follow each token's kept count (slots 0, 3, 6, 7, 12,
+                                   13, 19); for thresholded calls, whose `charges` then
+                                   hold the terms every active token adds */
 
 /* Stages of one call, in launch order (cfmoe_launch_stage). */
 #define CFMOE_STAGE_PREPARE 0 /* route, rotate, mask, grid quantisation */

@@ -266,3 +266,50 @@ def test_grouped_and_per_token_calls_agree_and_report_their_reads():
         blocks = hidden // 128
         assert report["issued_sketch_bytes"] == tiles * (64 * width * blocks + 4 * width * blocks)
         assert report["grouped_issued_matrix_macs"] == tiles * 2 * width * 16 * 128 * 3 * blocks
+
+
+@pytest.mark.parametrize("tokens,rank,score", [
+    (1, 32, "point"), (4, 16, "recovery-aware"), (15, 32, "point"), (16, 16, "point"),
+    (33, 64, "recovery-aware"),
+])
+def test_thresholded_read_statistics_follow_the_selection(tokens, rank, score):
+    """read_work of a thresholded call (fused, per-token and grouped schedules,
+    padded rows, tokens that keep nothing or the cap) against the reference's
+    pricing of the selection the call made (progressive.py:2189-2225)."""
+    layer = make_layer(hidden=512, width=256, experts=16, top_k=4, rank=rank, tokens=tokens, seed=131)
+    plan = compile_budget(hidden_size=512, expert_width=256, top_k=4, retention=0.2, screen_keep=0.625)
+    hidden = layer.hidden.clone()
+    if tokens > 1:
+        hidden[0] *= 50  # keeps the cap
+        hidden[1] = 0  # keeps nothing
+    probe = build(layer, plan, tokens, selection_score=score)
+    arguments = [v.to(DEVICE) for v in (hidden, layer.ids, layer.weights)]
+    probe(*arguments)
+    tau = float(probe.scores[0][:tokens].float().flatten().sort(descending=True).values[100 * tokens])
+    reader = build(layer, plan, tokens, selection_score=score, selection_threshold=max(tau, 1e-30))
+    padding = None
+    if tokens > 2:
+        padding = torch.zeros(tokens, dtype=torch.bool, device=DEVICE)
+        padding[2] = True
+    reader(*arguments, padding)
+    torch.cuda.synchronize()
+    work = reader.read_work.cpu().tolist()
+    active = torch.ones(tokens, dtype=torch.bool) if padding is None else ~padding.cpu()
+    kept = float(reader.selected[:tokens].cpu()[active].sum())
+    assert kept == float(reader.completed[:tokens].cpu()[active].sum())
+    count, n, h = float(active.sum()), plan.candidate_count, 512
+    geometry = reader.recovery_geometry is not None
+    residual = score != "point"
+    want = {
+        0: 6 * h * kept, 6: 6 * h * kept, 1: count * plan.native_read_bytes(),
+        3: 2 * rank * (count * n - kept + count * h), 7: 2 * rank * (count * n - kept + count * h),
+        4: (12 if geometry else 4) * count * n + 4 * count,
+        9: (12 if geometry else 4) * count * n + 32 * count,
+        5: count * plan.sketch_read_bytes(residual, sectors=False),
+        17: count * plan.sketch_read_bytes(residual), 10: count * h, 13: 2 * h * kept,
+        14: 2 * rank * count * n, 16: count if tokens >= 16 else 0.0, 19: count,
+    }
+    if tokens < 16:
+        want[12] = 4 * h * kept
+    assert {slot: work[slot] for slot in want} == want
+    assert 0 < kept < count * plan.final_count or tokens == 1
