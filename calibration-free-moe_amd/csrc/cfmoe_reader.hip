@@ -1924,6 +1924,11 @@ __device__ __forceinline__ void select_token(const SelectArgs &a, int t, bool wr
     }
   }
   auto valid = [&](int j) { return j < per && first + j < a.N; };
+  // a padded token's scores are all +0, every key one bin's: its first `want`
+  // candidates are the ties kept, without the passes (whose LDS atomics would
+  // all meet on that bin: select 22.2 us for 16 tokens, 3 of them padded,
+  // against 8.1 us)
+  const bool padded = !is_active(a.padding, t);
   int want = a.F;
   if (a.thresholded) {
     const uint32_t bound = __float_as_uint(*a.threshold + 0.0f);
@@ -1938,7 +1943,9 @@ __device__ __forceinline__ void select_token(const SelectArgs &a, int t, bool wr
   // radix passes find the want-th largest key: `prefix` holds its known
   // bits, `mask` which bits those are
   uint32_t prefix = 0, mask = 0;
-  if (want > 0) {
+  if (want > 0 && padded) {
+    mask = 0xffffffffu;
+  } else if (want > 0) {
 #pragma unroll
     for (int pass = 0; pass < 2; ++pass) {
       const int shift = pass == 0 ? 20 : 8;
@@ -2068,7 +2075,7 @@ __device__ __forceinline__ void select_token(const SelectArgs &a, int t, bool wr
   // the kept count's read statistics (integers, exact in FP64 in any order),
   // one slot per lane of wave 1 (a template argument: the test alone cost the
   // batch-1 calls that never charge 0.3 us)
-  if (kCharge && wave == 1 && lane < 7 && is_active(a.padding, t)) {
+  if (kCharge && wave == 1 && lane < 7 && !padded) {
     const int kept_slots[7] = {0, 6, 13, 12, 3, 7, 19};
     const int slot = kept_slots[lane];
     const double bytes = lane < 2 ? 6.0 * a.H : lane == 2 ? 2.0 * a.H : lane == 3 ? a.row_charge : -2.0 * a.R;
