@@ -1459,13 +1459,17 @@ __global__ __launch_bounds__(64 * kSmallWaves) void small_screen_kernel(SmallScr
 // and the up row tile I/16 + ct, over every rotation block. The blocks run in
 // split order; split s's partial is the fma chain over its blocks and the
 // estimate is ((part_0 + part_1) + part_2) + ... -- the arithmetic of
-// small_screen_kernel, with the partials kept in registers. The workgroup's waves share the tile's digit planes in LDS,
-// staged kStageAhead splits ahead (ring of kStageAhead + 1 buffers, one
-// barrier per split); a wave's block steps are loaded one split ahead, each
-// step's successor issued as soon as the step is used. The score epilogue
-// writes the projections and scores of the wave's 16 channels for the tile's
-// pairs. Workgroups past the tiles (one per token) write the zero projections
-// and scores of padded tokens and absent slots.
+// small_screen_kernel, with the partials kept in registers. The workgroup's waves share the
+// tile's digit planes in LDS, staged two blocks at a time, kStageAhead stages
+// ahead (ring of kStageAhead + 1 buffers, one barrier per stage); a wave's
+// block steps are loaded one stage ahead, each step's successor issued as soon
+// as the step is used. Staging two blocks whatever a split holds keeps wide
+// layers at four workgroups per CU (a staged split of three or four blocks held
+// two: H = 2816 recovery-aware at 24 tokens 68 -> 41 us with the compact
+// epilogue, H = 4096 at 48 tokens 124 -> 103 us). The score epilogue writes the
+// projections and scores of the wave's 16 channels for the tile's pairs.
+// Workgroups past the tiles (one per token) write the zero projections and
+// scores of padded tokens and absent slots.
 
 constexpr int kFusedWaves = 4;
 constexpr int kFusedThreads = 64 * kFusedWaves;
@@ -1505,22 +1509,39 @@ struct FusedScreenArgs {
   int gelu, point;
 };
 
-template <bool kGh5, int kSpan>
+// Rotation blocks staged together, whatever a split's blocks.
+constexpr int kStageBlocks = 2;
+constexpr int kMaxBlocks = kMaxSpan * kMaxSplits;
+
+// kPaired: two-block splits (1024 < H <= 2048), a stage each; otherwise the
+// splits end where the block index says, and the tables hold kMaxBlocks.
+template <bool kGh5, bool kPaired>
 struct FusedShared {
-  alignas(16) int8_t digits[kStageBuffers][kSpan][3][kPairTile][kDigitStride];
-  // the split's FP16 scales (and residual scales) of the workgroup's gate and
-  // up row tiles (one of each per wave): entry kScaleBlock (kSpan kind + bl)
-  // + 4 kFusedWaves up + 4 w + q holds rows 4q .. 4q + 3 of wave w's row tile
-  uint2 scales[kStageBuffers][(kGh5 ? 2 : 1) * kSpan * kScaleBlock];
-  int qsum[kSpan * kMaxSplits][kPairTile];  // blocks x pairs
-  int shift[kSpan * kMaxSplits][kPairTile];
-  float norm2[kGh5 ? kSpan * kMaxSplits : 1][kPairTile];
+  static constexpr int kTableBlocks = kPaired ? kStageBlocks * kMaxSplits : kMaxBlocks;
+  alignas(16) int8_t digits[kStageBuffers][kStageBlocks][3][kPairTile][kDigitStride];
+  // the stage's FP16 scales (and residual scales) of the workgroup's gate and
+  // up row tiles (one of each per wave): entry kScaleBlock (kStageBlocks kind
+  // + bl) + 4 kFusedWaves up + 4 w + q holds rows 4q .. 4q + 3 of wave w's row tile
+  uint2 scales[kStageBuffers][(kGh5 ? 2 : 1) * kStageBlocks * kScaleBlock];
+  int qsum[kTableBlocks][kPairTile];  // blocks x pairs
+  int shift[kTableBlocks][kPairTile];
+  float norm2[kGh5 ? kTableBlocks : 1][kPairTile];
   int pair_token[kPairTile], pair_slot[kPairTile];
 };
 
-template <bool kGh5, int kSpan>
-__global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(kSpan == kNarrowSpan ? (kGh5 ? 3 : 5) : 2))) void fused_screen_kernel(FusedScreenArgs a) {
-  __shared__ FusedShared<kGh5, kSpan> sh;
+// Pairs up to which the score epilogue hands a wave's (pair, channel) items
+// out one per lane through LDS: a tile of n pairs then takes ceil(n / 4)
+// rounds of one score, not four scores in the lanes of its n columns (a
+// 16-token recovery-aware call has 1.5 pairs per tile: 33 -> 25 us). Point scores are
+// cheap: they take this way only where one round does. The values of twelve
+// pairs fit a wave's quarter of a free staging buffer.
+template <bool kGh5>
+constexpr int kCompactPairs = kGh5 ? 12 : 4;
+
+template <bool kGh5, bool kPaired>
+__global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(kPaired && !kGh5 ? 5 : 4))) void fused_screen_kernel(FusedScreenArgs a) {
+  using Shared = FusedShared<kGh5, kPaired>;
+  __shared__ Shared sh;
   // (the wave index through a scalar register: every wave-uniform address
   // term below is then scalar arithmetic, not a vector instruction per lane)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1540,25 +1561,25 @@ __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(k
   const int e = load_uniform(a.group_experts + z);
   const int count = load_uniform(a.group_counts + z);
   const int pp = lane % 16, k0 = 16 * (lane / 16), row_in_tile = 4 * (lane / 16);
-  const int span = a.span, splits = a.splits;
+  const int stages = (B + kStageBlocks - 1) / kStageBlocks;
   // the wave's trit planes: gate row tile cc, up row tile CT + cc (a
   // wave-uniform row-tile base, lane l's 8 bytes at 8 l); the scales come
   // with the staging
   const uint2 *planes = a.planes + static_cast<long>(e) * B * RT * 64;
   const uint16_t *stats = a.stats + static_cast<long>(e) * B * 4 * a.I;
   auto load_step = [&](int s, int bl, int up) {
-    const int b = min(s * span + min(bl, span - 1), B - 1);  // past H: a repeat, unused
+    const int b = min(kStageBlocks * s + bl, B - 1);  // past H: a repeat, unused
     const int rt = up ? CT + cc : cc;
     const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(
         buffer_resource(planes + (b * RT + rt) * 64, 64 * 8), lane * 8, 0, 0);
     return make_uint2(v.x, v.y);
   };
-  // split 0's steps in flight while the tile is staged; each step's
-  // successor (the next split's) is loaded into its registers as soon as the
+  // stage 0's steps in flight while the tile is staged; each step's
+  // successor (the next stage's) is loaded into its registers as soon as the
   // step is expanded
-  uint2 step[kSpan][2];
+  uint2 step[kStageBlocks][2];
 #pragma unroll
-  for (int bl = 0; bl < kSpan; ++bl)
+  for (int bl = 0; bl < kStageBlocks; ++bl)
 #pragma unroll
     for (int up = 0; up < 2; ++up) step[bl][up] = load_step(0, bl, up);
 
@@ -1579,9 +1600,8 @@ __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(k
   }
   __syncthreads();
   // thread tid's (block, pair) entries: tid = 16 b + p, then 16 (b + 16) + p
-  // at span 4 (up to 32 blocks); loaded with the first split's staging,
-  // stored after it
-  constexpr int kTableBlocks = kSpan * kMaxSplits;
+  // with up to 32 blocks; loaded with the first stage's staging, stored after it
+  constexpr int kTableBlocks = Shared::kTableBlocks;
   constexpr int kTableRounds = (kTableBlocks * kPairTile + kFusedThreads - 1) / kFusedThreads;
   const int tp = tid % kPairTile;
   int qsum_value[kTableRounds], shift_value[kTableRounds];
@@ -1596,26 +1616,26 @@ __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(k
     shift_value[r] = load_global(a.qexp + table_cell);
     norm2_value[r] = kGh5 ? load_global(a.norm2 + table_cell) : 0.0f;
   }
-  // staging of split s: rows (block, digit, pair) of 128 bytes, 16 bytes per
+  // staging of stage s: rows (block, digit, pair) of 128 bytes, 16 bytes per
   // thread and item. Every load is unconditional and in bounds: a pair past
   // the count reads the tile's first pair (its MFMA B column feeds only that
-  // pair's unused results) and a block past H or the split reads block B - 1
+  // pair's unused results) and a block past H reads block B - 1
   // (never used)
-  constexpr int kStageRows = kSpan * 3 * kPairTile;
-  constexpr int kStageItems = kStageRows * 8;  // uint4 per split
+  constexpr int kStageRows = kStageBlocks * 3 * kPairTile;
+  constexpr int kStageItems = kStageRows * 8;  // uint4 per stage
   constexpr int kStagePerThread = kStageItems / kFusedThreads;
   static_assert(kStageItems % kFusedThreads == 0, "staging items per thread");
   // an item's block (item / 384) is wave-uniform: 384 items are six waves
   static_assert((8 * 3 * kPairTile) % kWave == 0, "staging blocks change at wave boundaries");
   // Thread i also loads scale entry i (see FusedShared; threads past the
   // entries repeat entry i % entries, and a row tile past the channels reads
-  // the last one). Lane offsets are fixed; per split the entries come through
-  // a buffer resource over the split's blocks to the expert's last, so an
+  // the last one). Lane offsets are fixed; per stage the entries come through
+  // a buffer resource over the stage's blocks to the expert's last, so an
   // entry of a block past the expert (never used) reads zeros
-  constexpr int kScaleEntries = (kGh5 ? 2 : 1) * kSpan * kScaleBlock;
+  constexpr int kScaleEntries = (kGh5 ? 2 : 1) * kStageBlocks * kScaleBlock;
   static_assert(kScaleEntries <= kFusedThreads, "one scale entry per thread at most");
   const int sentry = tid % kScaleEntries;
-  const int sk = kGh5 ? sentry / (kScaleBlock * kSpan) : 0, sbl = (sentry / kScaleBlock) % kSpan;
+  const int sk = kGh5 ? sentry / (kScaleBlock * kStageBlocks) : 0, sbl = (sentry / kScaleBlock) % kStageBlocks;
   const int within = sentry % kScaleBlock;
   const int sup = within / (kFusedWaves * kScaleQuads), sw = (within / kScaleQuads) % kFusedWaves;
   const int stile = (sup ? CT : 0) + min(group * kFusedWaves + sw, CT - 1);
@@ -1634,10 +1654,10 @@ __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(k
 #pragma unroll
     for (int j = 0; j < kStagePerThread; ++j) {
       const int bl = (kWave * wave + j * kFusedThreads) / (8 * 3 * kPairTile);
-      const int b = min(s * span + bl, B - 1);
+      const int b = min(kStageBlocks * s + bl, B - 1);
       held[j] = buffer_load16(buffer_resource(a.digits + b * 384, (a.T * B - b) * 384), stage_offset[j]);
     }
-    const int first = min(s * span, B);  // B for the prefetch past the last split: no records
+    const int first = min(kStageBlocks * s, B);  // B for the prefetch past the last stage: no records
     const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(
         buffer_resource(stats + first * 4 * a.I, (B - first) * 8 * a.I), scale_offset, 0, 0);
     scale = make_uint2(v.x, v.y);
@@ -1653,7 +1673,7 @@ __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(k
   };
   uint4 held[kStagePerThread];
   uint2 held_scale;
-  static_assert(kStageAhead == 1, "one split staged ahead");
+  static_assert(kStageAhead == 1, "one stage ahead");
   stage_load(0, held, held_scale);
   // (no store moves above this point: the table and staging loads are all
   // issued before the first wait)
@@ -1671,30 +1691,47 @@ __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(k
   stage_store(0, held, held_scale);
   __syncthreads();
 
-  float est[2][4] = {}, var[2][4] = {};
-  // splits from ceil(B / span) on hold no block (B = 9: splits 5-7 of span
-  // 2): their zero partials are added after the loop, so every split in it
-  // has a first block below B
-  const int live_splits = (B + span - 1) / span;
-  for (int s = 0; s < live_splits; ++s) {
+  // a split's partial is the fma chain over its blocks from +0, the estimate
+  // the partials' sum in split order (from -0, so that the first is taken as
+  // it is)
+  float est[2][4], var[2][4], part[2][4], vpart[2][4];
+#pragma unroll
+  for (int up = 0; up < 2; ++up)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      est[up][r] = var[up][r] = -0.0f;
+      part[up][r] = vpart[up][r] = 0.0f;
+    }
+  auto end_split = [&] {
+#pragma unroll
+    for (int up = 0; up < 2; ++up)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        est[up][r] = est[up][r] + part[up][r];
+        part[up][r] = 0.0f;
+        if (kGh5) {
+          var[up][r] = var[up][r] + vpart[up][r];
+          vpart[up][r] = 0.0f;
+        }
+      }
+  };
+  int split_left = a.span;  // blocks left in the split
+  for (int s = 0; s < stages; ++s) {
     const int buffer = s % kStageBuffers;
-    // split s + kStageAhead's digits go to the buffer split s - 1 used, which
+    // stage s + kStageAhead's digits go to the buffer stage s - 1 used, which
     // every wave finished before the last barrier
     stage_load(s + kStageAhead, held, held_scale);
-    // (a split's first block, always below B, starts the chains from zero
-    // as an fma operand; a later block past the split or H leaves them)
-    float part[2][4], vpart[2][4];
 #pragma unroll
-    for (int bl = 0; bl < kSpan; ++bl) {
-      const int b = s * span + bl;
-      const bool live_block = bl == 0 || (bl < span && b < B);
+    for (int bl = 0; bl < kStageBlocks; ++bl) {
+      const int b = kStageBlocks * s + bl;
+      const bool live_block = bl == 0 || b < B;
       const int start = sh.qsum[min(b, B - 1)][pp], shift = sh.shift[min(b, B - 1)][pp];
       const float n2 = kGh5 ? sh.norm2[kGh5 ? min(b, B - 1) : 0][pp] : 0.0f;
       auto operand = [&](int h, int d) {
         return *reinterpret_cast<const v4i *>(&sh.digits[buffer][bl][d][pp][64 * h + k0]);
       };
       // gate and up row tiles share each B operand read; the expanded step's
-      // registers take its successor (a repeat past the last split)
+      // registers take its successor (a repeat past the last stage)
       v4i a0[2], a1[2];
 #pragma unroll
       for (int up = 0; up < 2; ++up) {
@@ -1703,7 +1740,7 @@ __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(k
         // (the successor load stays below the expansion, so it can take the
         // step's own registers: no copy round the loop waits for it)
         asm volatile("" ::"v"(a0[up]), "v"(a1[up]) : "memory");
-        step[bl][up] = load_step(s + 1 < live_splits ? s + 1 : s, bl, up);
+        step[bl][up] = load_step(s + 1 < stages ? s + 1 : s, bl, up);
       }
       if (!live_block) continue;
       v4i acc[2];
@@ -1712,33 +1749,33 @@ __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(k
       for (int up = 0; up < 2; ++up) {
         const int entry = kScaleBlock * bl + kFusedWaves * kScaleQuads * up + kScaleQuads * wave + (lane >> 4);
         const uint2 scale = sh.scales[buffer][entry];
-        const uint2 residual = kGh5 ? sh.scales[buffer][kScaleBlock * kSpan + entry] : make_uint2(0u, 0u);
+        const uint2 residual = kGh5 ? sh.scales[buffer][kScaleBlock * kStageBlocks + entry] : make_uint2(0u, 0u);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int sum = acc[up][r];
           const float dot = ldexpf(static_cast<float>(sum), shift);
           const uint32_t sw = r < 2 ? scale.x : scale.y;
-          part[up][r] = fmaf(dot, half_at(sw, r & 1), bl == 0 ? 0.0f : part[up][r]);
+          part[up][r] = fmaf(dot, half_at(sw, r & 1), part[up][r]);
           if (kGh5) {
             const uint32_t rw = r < 2 ? residual.x : residual.y;
-            vpart[up][r] = fmaf(half_at(rw, r & 1), n2, bl == 0 ? 0.0f : vpart[up][r]);
+            vpart[up][r] = fmaf(half_at(rw, r & 1), n2, vpart[up][r]);
           }
         }
       }
-    }
-#pragma unroll
-    for (int up = 0; up < 2; ++up)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        est[up][r] = s == 0 ? part[up][r] : est[up][r] + part[up][r];
-        if (kGh5) var[up][r] = s == 0 ? vpart[up][r] : var[up][r] + vpart[up][r];
+      if (!kPaired && (--split_left == 0 || b + 1 == B)) {
+        end_split();
+        split_left = a.span;
       }
-    if (s + 1 < live_splits) {
+    }
+    if (kPaired) end_split();
+    if (s + 1 < stages) {
       stage_store((s + kStageAhead) % kStageBuffers, held, held_scale);
       __syncthreads();
     }
   }
-  for (int s = live_splits; s < splits; ++s)
+  // splits from ceil(B / span) on hold no block (B = 9: splits 5-7 of span
+  // 2): they add zero partials, after which no estimate is -0
+  if ((B + a.span - 1) / a.span < a.splits)
 #pragma unroll
     for (int up = 0; up < 2; ++up)
 #pragma unroll
@@ -1746,10 +1783,45 @@ __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(k
         est[up][r] = est[up][r] + 0.0f;
         if (kGh5) var[up][r] = var[up][r] + 0.0f;
       }
-  // ---- score epilogue: lane (pair pp, channels c .. c + 3)
+  // ---- score epilogue
   if (!working) return;
   if (a.tile_masks && lane < kRowTile)
     a.tile_masks[static_cast<long>(z) * a.I + kRowTile * ct + lane] = 0u;
+  if (count <= kCompactPairs<kGh5>) {
+    // one (pair, channel) item per lane: the wave's values through its quarter
+    // of the staging buffer the last stage left free (every wave finished with
+    // it before the last barrier; a wave's LDS operations complete in order)
+    constexpr int kPlane = kCompactPairs<kGh5> * kRowTile;
+    static_assert(sizeof(sh.digits[0]) >= kFusedWaves * (kGh5 ? 4 : 2) * kPlane * sizeof(float), "epilogue values");
+    float *values = reinterpret_cast<float *>(&sh.digits[stages % kStageBuffers][0][0][0][0]) +
+                    wave * (kGh5 ? 4 : 2) * kPlane;
+    if (pp < count)
+#pragma unroll
+      for (int up = 0; up < 2; ++up) {
+        float *row = values + up * kPlane + kRowTile * pp + row_in_tile;
+        *reinterpret_cast<float4 *>(row) = make_float4(est[up][0], est[up][1], est[up][2], est[up][3]);
+        if (kGh5)
+          *reinterpret_cast<float4 *>(row + 2 * kPlane) =
+              make_float4(var[up][0], var[up][1], var[up][2], var[up][3]);
+      }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int c = kRowTile * ct + pp;
+    const long channel = static_cast<long>(e) * a.I + c;
+    const float norm = load_global(a.norms + channel);
+    const float alpha = a.geometry ? load_global(a.geometry + 2 * channel) : 0.0f;
+    const float beta = a.geometry ? load_global(a.geometry + 2 * channel + 1) : 0.0f;
+    for (int p = lane / kRowTile; p < count; p += kWave / kRowTile) {
+      const int token = sh.pair_token[p], slot = sh.pair_slot[p];
+      const float *value = values + kRowTile * p + pp;
+      score_one<kGh5>(a, token, slot, c, value[0], value[kPlane], kGh5 ? value[2 * kPlane] : 0.0f,
+                      kGh5 ? value[3 * kPlane] : 0.0f, norm, load_global(a.weights + token * a.K + slot), alpha,
+                      beta);
+    }
+    return;
+  }
+  // lane (pair pp, channels c .. c + 3)
   if (pp >= count) return;
   // (the score's inputs here: held across the splits they would cost a wave per SIMD)
   const int c = kRowTile * ct + row_in_tile;
@@ -3857,15 +3929,12 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
       fs.gelu = gelu;
       fs.point = !gh5;
       const unsigned blocks = static_cast<unsigned>(fs.tile_items + tokens);
-      const bool narrow = s.span <= kNarrowSpan;
-      if (gh5 && narrow)
-        hipLaunchKernelGGL((fused_screen_kernel<true, kNarrowSpan>), dim3(blocks), dim3(kFusedThreads), 0, stream, fs);
-      else if (gh5)
-        hipLaunchKernelGGL((fused_screen_kernel<true, kMaxSpan>), dim3(blocks), dim3(kFusedThreads), 0, stream, fs);
-      else if (narrow)
-        hipLaunchKernelGGL((fused_screen_kernel<false, kNarrowSpan>), dim3(blocks), dim3(kFusedThreads), 0, stream, fs);
-      else
-        hipLaunchKernelGGL((fused_screen_kernel<false, kMaxSpan>), dim3(blocks), dim3(kFusedThreads), 0, stream, fs);
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kFusedThreads), 0, stream, fs);
+      };
+      const bool paired = s.span == kStageBlocks;
+      if (gh5) launch(paired ? fused_screen_kernel<true, true> : fused_screen_kernel<true, false>);
+      else launch(paired ? fused_screen_kernel<false, true> : fused_screen_kernel<false, false>);
       if ((rc = check_launch("screen"))) return rc;
     } else if (stages & (1u << CFMOE_STAGE_SCREEN)) {
       const SmallScreenArgs ss = small_screen_args(s, dims, weights, workspace, padding, tokens);
