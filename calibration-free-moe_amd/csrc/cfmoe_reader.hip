@@ -434,7 +434,13 @@ __device__ inline RouteShared route_layout(char *lds, int pairs, int experts) {
   return r;
 }
 
-template <int kPrepareThreads, bool kIds64, bool kWeights16>
+// The routing block runs once, alone on its CU, so its instructions come cold
+// from the caches: it is compiled for the pairs a thread holds (kBatch: 1, 2
+// or 8, see launch_prepare) rather than for eight with most of them masked
+// off, the counters are cleared before the first barrier, a pair counts its
+// expert where it is placed, and the pairs' ranks are formed between the two
+// halves of the experts' scan: four barriers.
+template <int kPrepareThreads, int kBatch, bool kIds64, bool kWeights16>
 __device__ __forceinline__ void route_and_group(const PrepareArgs &a, const RouteShared &shared,
                                                 int *scratch) {
   constexpr int kPrepareWaves = kPrepareThreads / 64;
@@ -454,12 +460,10 @@ __device__ __forceinline__ void route_and_group(const PrepareArgs &a, const Rout
                       : load_global(static_cast<const float *>(a.router_weights) + q);
   };
   // Each thread's first kBatch pairs p = tid + kPrepareThreads q (all of
-  // them up to 8 pairs per thread: the host runs 1024 threads from 1024
-  // pairs unless the experts' LDS lists are too large): the raw ids, the
-  // router weights and the pairs' tokens' padding flags in one round trip,
-  // every load unconditional (clamped index; the formats are template
-  // arguments; a padding source of zero bytes reads zero: active)
-  constexpr int kBatch = 8;
+  // them unless the experts' LDS lists are too large for 1024 threads): the
+  // raw ids, the router weights and the pairs' tokens' padding flags in one
+  // round trip, every load unconditional (clamped index; the formats are
+  // template arguments; a padding source of zero bytes reads zero: active)
   const __amdgpu_buffer_rsrc_t padding = buffer_resource(a.padding_source, a.padding_bytes);
   auto raw_id_of = [&](int p) {
     if (kIds64) {
@@ -485,6 +489,8 @@ __device__ __forceinline__ void route_and_group(const PrepareArgs &a, const Rout
   }
   // (every load above is issued before the first is used)
   asm volatile("" ::: "memory");
+  for (int e = tid; e < a.E; e += kPrepareThreads) counts[e] = 0;
+  for (int i = tid; i < kPrepareWaves * a.E; i += kPrepareThreads) shared.wave_counts[i] = 0;
   int active_tokens = 0;  // tokens counted at their slot 0
 #pragma unroll
   for (int q = 0; q < kBatch; ++q) {
@@ -542,6 +548,7 @@ __device__ __forceinline__ void route_and_group(const PrepareArgs &a, const Rout
     a.ids[t * K + rank] = id;
     a.weights[t * K + rank] = w;
     sorted[t * K + rank] = static_cast<int16_t>(active ? id : -1);
+    if (active && id >= 0) atomicAdd(&counts[id], 1);
   };
 #pragma unroll
   for (int q = 0; q < kBatch; ++q) {
@@ -555,62 +562,29 @@ __device__ __forceinline__ void route_and_group(const PrepareArgs &a, const Rout
   for (int p = pairs + tid; p < padded; p += kPrepareThreads) sorted[p] = -1;
   __syncthreads();
   // Expert-major grouping as a counting sort by expert, stable in pair order:
-  // (1) per-expert counts; (2) one scan of packed (members, tiles) gives each
-  // expert its member start and first tile z_e, and its tiles are emitted;
-  // (3) wave w ranks the pairs of its contiguous range among the earlier
-  // pairs of the same expert (a match of equal experts from one ballot per id
-  // bit, 64 pairs at a time, running per-expert counts of the wave); (4) a
-  // pair's final slot is 16 z_e + its rank within its wave's range + the
+  // (1) the experts' counts (taken above) go through one scan of packed
+  // (members, tiles), which gives each expert its first tile z_e, and its tiles
+  // are emitted; (2) wave w ranks the pairs of its contiguous range among the
+  // earlier pairs of the same expert (a match of equal experts from one ballot
+  // per id bit, 64 pairs at a time, running per-expert counts of the wave);
+  // (3) a pair's final slot is 16 z_e + its rank within its wave's range + the
   // counts of the waves before. O(pairs log E), whatever the skew.
-  for (int e = tid; e <= a.E; e += kPrepareThreads) counts[e] = 0;
-  for (int i = tid; i < kPrepareWaves * a.E; i += kPrepareThreads) shared.wave_counts[i] = 0;
-  __syncthreads();
-  for (int p = tid; p < pairs; p += kPrepareThreads) {
-    const int e = sorted[p];
-    if (e >= 0) atomicAdd(&counts[e], 1);
-  }
-  __syncthreads();
+  const int wave = tid >> 6, lane = tid & 63;
   // thread i owns the experts [i per, (i + 1) per)
   const int per = (a.E + kPrepareThreads - 1) / kPrepareThreads;
   const int first = min(a.E, tid * per), last = min(a.E, first + per);
-  int members = 0, tiles = 0;
-  for (int e = first; e < last; ++e) {
-    members += counts[e];
-    tiles += (counts[e] + kGroupPairs - 1) / kGroupPairs;
-  }
-  int packed_total;  // members and tiles are below 2^16 (pairs <= 8192)
-  const int packed = block_exclusive(members | (tiles << 16), scratch, &packed_total);
-  const int total_tiles = packed_total >> 16;
-  // the per-tile read charges (integers, exact in FP64), issued as soon as
-  // the tile count is known
-  if (account && total_tiles > 0) {
-    const double tile_count = static_cast<double>(total_tiles);
-    if (tid == 32 && a.tile_sketch_bytes != 0.0) atomicAdd(a.read_work + 11, tile_count * a.tile_sketch_bytes);
-    if (tid == 33 && a.tile_screen_macs != 0.0) atomicAdd(a.read_work + 15, tile_count * a.tile_screen_macs);
-    if (tid == 34 && a.tile_row_bytes != 0.0) atomicAdd(a.read_work + 12, tile_count * a.tile_row_bytes);
-  }
+  int packed_here = 0;  // members and tiles, below 2^16 each (pairs <= 8192)
+  for (int e = first; e < last; ++e)
+    packed_here += counts[e] | ((counts[e] + kGroupPairs - 1) / kGroupPairs) << 16;
+  const int inclusive = wave_inclusive(packed_here);
+  int *wave_packed = scratch + 16;
+  if (lane == 63) wave_packed[wave] = inclusive;
+  const int chunks = (pairs + 63) / 64;
+  const int per_wave = (chunks + kPrepareWaves - 1) / kPrepareWaves;
+  int16_t *local_rank = routed;
   {
-    int start = packed & 0xffff, z = packed >> 16;
-    for (int e = first; e < last; ++e) {
-      const int count = counts[e];
-      base[e] = start | (z << 16);
-      for (int first_pair = 0; first_pair < count; first_pair += kGroupPairs) {
-        a.group_experts[z] = e;
-        a.group_starts[z] = kGroupPairs * z;
-        a.group_counts[z] = min(kGroupPairs, count - first_pair);
-        ++z;
-      }
-      start += count;
-    }
-    if (tid == kPrepareThreads - 1) base[a.E] = packed_total & 0xffff;
-  }
-  {
-    const int wave = tid >> 6, lane = tid & 63;
-    const int chunks = (pairs + 63) / 64;
-    const int per_wave = (chunks + kPrepareWaves - 1) / kPrepareWaves;
     const int bits = a.E > 1 ? 32 - __builtin_clz(static_cast<unsigned>(a.E - 1)) : 1;
     int16_t *counted = shared.wave_counts + wave * a.E;
-    int16_t *local_rank = routed;
     for (int c = wave * per_wave; c < min(chunks, (wave + 1) * per_wave); ++c) {
       const int p = 64 * c + lane;
       const int e = p < pairs ? sorted[p] : -1;
@@ -629,19 +603,54 @@ __device__ __forceinline__ void route_and_group(const PrepareArgs &a, const Rout
         if (lane == __builtin_ctzll(peers)) counted[e] = static_cast<int16_t>(before + __popcll(peers));
       }
     }
-    __syncthreads();
-    for (int p = tid; p < pairs; p += kPrepareThreads) {
-      const int e = sorted[p];
-      if (e < 0) continue;
-      const int owner = (p / 64) / per_wave;
-      int rank = local_rank[p];
-      for (int v = 0; v < owner; ++v) rank += shared.wave_counts[v * a.E + e];
-      const int at = kGroupPairs * (base[e] >> 16) + rank;
-      a.group_pairs[at] = p;
-      a.pair_tiles[p] = at;
+  }
+  __syncthreads();
+  int packed = inclusive - packed_here, packed_total = 0;
+#pragma unroll
+  for (int w = 0; w < kPrepareWaves; ++w) {
+    const int v = wave_packed[w];
+    packed += w < wave ? v : 0;
+    packed_total += v;
+  }
+  const int total_tiles = packed_total >> 16;
+  // the per-tile read charges (integers, exact in FP64), issued as soon as
+  // the tile count is known
+  if (account && total_tiles > 0) {
+    const double tile_count = static_cast<double>(total_tiles);
+    if (tid == 32 && a.tile_sketch_bytes != 0.0) atomicAdd(a.read_work + 11, tile_count * a.tile_sketch_bytes);
+    if (tid == 33 && a.tile_screen_macs != 0.0) atomicAdd(a.read_work + 15, tile_count * a.tile_screen_macs);
+    if (tid == 34 && a.tile_row_bytes != 0.0) atomicAdd(a.read_work + 12, tile_count * a.tile_row_bytes);
+  }
+  int z = packed >> 16;
+  for (int e = first; e < last; ++e) {
+    const int count = counts[e];
+    base[e] = z;
+    for (int first_pair = 0; first_pair < count; first_pair += kGroupPairs) {
+      a.group_experts[z] = e;
+      a.group_starts[z] = kGroupPairs * z;
+      a.group_counts[z] = min(kGroupPairs, count - first_pair);
+      ++z;
     }
   }
   if (tid == 0) *a.group_total = total_tiles;
+  __syncthreads();
+  for (int p = tid; p < pairs; p += kPrepareThreads) {
+    const int e = sorted[p];
+    if (e < 0) continue;
+    const int owner = (p / 64) / per_wave;
+    int rank = local_rank[p];
+    // (four waves' counts at a time, so their reads are in flight together)
+    for (int v = 0; v < owner; v += 4) {
+      int before[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) before[u] = shared.wave_counts[min(v + u, kPrepareWaves - 1) * a.E + e];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) rank += v + u < owner ? before[u] : 0;
+    }
+    const int at = kGroupPairs * base[e] + rank;
+    a.group_pairs[at] = p;
+    a.pair_tiles[p] = at;
+  }
 }
 
 // One-token routing on one wave, in one round trip and without barriers (the
@@ -908,7 +917,7 @@ __device__ __forceinline__ void store_cell(const PrepareArgs &a, long cell, cons
   row[320 + lane] = static_cast<int8_t>(d2);
 }
 
-template <int kPrepareThreads>
+template <int kPrepareThreads, int kBatch>
 __global__ __launch_bounds__(kPrepareThreads) void prepare_kernel(PrepareArgs a) {
   constexpr int kPrepareWaves = kPrepareThreads / 64;
   // block 0 routes and groups (the longest block, dispatched first)
@@ -921,11 +930,11 @@ __global__ __launch_bounds__(kPrepareThreads) void prepare_kernel(PrepareArgs a)
   if (a.route && blockIdx.x == 0) {
     const RouteShared shared = route_layout(route_lds, a.T * a.K, a.E);
     if (a.flags & CFMOE_IDS_INT64) {
-      if (a.flags & CFMOE_WEIGHTS_BF16) route_and_group<kPrepareThreads, true, true>(a, shared, route_scratch);
-      else route_and_group<kPrepareThreads, true, false>(a, shared, route_scratch);
+      if (a.flags & CFMOE_WEIGHTS_BF16) route_and_group<kPrepareThreads, kBatch, true, true>(a, shared, route_scratch);
+      else route_and_group<kPrepareThreads, kBatch, true, false>(a, shared, route_scratch);
     } else {
-      if (a.flags & CFMOE_WEIGHTS_BF16) route_and_group<kPrepareThreads, false, true>(a, shared, route_scratch);
-      else route_and_group<kPrepareThreads, false, false>(a, shared, route_scratch);
+      if (a.flags & CFMOE_WEIGHTS_BF16) route_and_group<kPrepareThreads, kBatch, false, true>(a, shared, route_scratch);
+      else route_and_group<kPrepareThreads, kBatch, false, false>(a, shared, route_scratch);
     }
     return;
   }
@@ -1131,7 +1140,7 @@ __device__ void score_absent_slots(const Args &a, int t, int threads) {
         a.variances[base + a.N] = 0.0f;
       }
       a.scores[flat] = cfm_score(0.0f, 0.0f, 0.0f, 0.0f, 0.0f, a.weights[t * a.K + k], 0.0f, 0.0f,
-                                 a.gelu != 0, a.point != 0);
+                                 a.gelu != 0, !kGh5);
     }
   }
 }
@@ -1194,7 +1203,7 @@ __device__ __forceinline__ void score_four(const Args &a, int token, int slot, i
 #pragma unroll
   for (int r = 0; r < 4; ++r)
     score[r] = cfm_score(gate[r], up[r], gate_var[r], up_var[r], in.norm[r], in.weight, in.alpha[r],
-                         in.beta[r], a.gelu != 0, a.point != 0);
+                         in.beta[r], a.gelu != 0, !kGh5);
   *reinterpret_cast<float4 *>(a.scores + static_cast<long>(token) * a.N + static_cast<long>(slot) * a.I + c) =
       make_float4(score[0], score[1], score[2], score[3]);
 }
@@ -1212,7 +1221,7 @@ __device__ __forceinline__ void score_one(const Args &a, int token, int slot, in
     a.variances[base + a.N] = up_var;
   }
   a.scores[static_cast<long>(token) * a.N + static_cast<long>(slot) * a.I + c] =
-      cfm_score(gate, up, gate_var, up_var, norm, weight, alpha, beta, a.gelu != 0, a.point != 0);
+      cfm_score(gate, up, gate_var, up_var, norm, weight, alpha, beta, a.gelu != 0, !kGh5);
 }
 
 // ---------------------------------------------------------------------------
@@ -3640,12 +3649,19 @@ int launch_prepare(const Shape &s, const cfmoe_dims *d, const cfmoe_weights *w,
   const int cell_blocks = (a.cells + threads / 64 - 1) / (threads / 64);
   // (a one-token call routes on one wave, without the LDS lists)
   const long lds = route && tokens > 1 ? route_lds_bytes(pairs, d->experts, threads / 64) : 0;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(cell_blocks + (route ? 1 : 0)), dim3(threads), static_cast<unsigned>(lds), stream, a);
+  };
+  // the routing block's pairs per thread (its loops take any further ones)
+  const int batch = (pairs + threads - 1) / threads;
   if (wide)
-    hipLaunchKernelGGL(prepare_kernel<kWidePrepareThreads>, dim3(cell_blocks + 1), dim3(threads),
-                       static_cast<unsigned>(lds), stream, a);
+    launch(batch <= 1   ? prepare_kernel<kWidePrepareThreads, 1>
+           : batch <= 2 ? prepare_kernel<kWidePrepareThreads, 2>
+                        : prepare_kernel<kWidePrepareThreads, 8>);
   else
-    hipLaunchKernelGGL(prepare_kernel<kPrepareThreads>, dim3(cell_blocks + (route ? 1 : 0)), dim3(threads),
-                       static_cast<unsigned>(lds), stream, a);
+    launch(batch <= 1   ? prepare_kernel<kPrepareThreads, 1>
+           : batch <= 2 ? prepare_kernel<kPrepareThreads, 2>
+                        : prepare_kernel<kPrepareThreads, 8>);
   return check_launch("prepare");
 }
 
