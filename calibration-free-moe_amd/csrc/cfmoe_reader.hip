@@ -1967,18 +1967,18 @@ __device__ __forceinline__ void select_token(const SelectArgs &a, int t, bool wr
   if (a.tile_masks && tid < a.K) slot_tiles[tid] = a.pair_tiles[t * a.K + tid];
   for (int i = tid; i < 2 * kSelectWideSlots; i += kSelectThreads) (&wide[0][0])[i] = 0;
   if (tid < kSelectLastSlots) last[tid] = 0;
-  const int per = (a.N + kSelectThreads - 1) / kSelectThreads;
+  constexpr int per = kKeys;
   const int first = tid * per;
   // keys: every load issued unconditionally (absent keys read a zero), four
-  // or two at a time when the thread's run allows (N is a multiple of 16, so
-  // a run of 4 or 2 keys is inside the row or wholly past it)
+  // or two at a time (N is a multiple of 16, so a run of 4 or 2 keys is inside
+  // the row or wholly past it)
   uint32_t key[kKeys];
   const float *row = a.scores + static_cast<long>(t) * a.N;
   auto normal = [](uint32_t bits) { return __float_as_uint(__uint_as_float(bits) + 0.0f); };
-  if (per % 4 == 0) {
+  if constexpr (per % 4 == 0) {
 #pragma unroll
     for (int j = 0; j < kKeys; j += 4) {
-      const bool present = j < per && first + j < a.N;
+      const bool present = first + j < a.N;
       const uint4 v =
           load_global(present ? reinterpret_cast<const uint4 *>(row + first + j) : &kZeroVector);
       key[j] = normal(v.x);
@@ -1986,25 +1986,18 @@ __device__ __forceinline__ void select_token(const SelectArgs &a, int t, bool wr
       key[j + 2] = normal(v.z);
       key[j + 3] = normal(v.w);
     }
-  } else if (per % 2 == 0) {
+  } else {
+    static_assert(per % 2 == 0, "keys per thread");
 #pragma unroll
     for (int j = 0; j < kKeys; j += 2) {
-      const bool present = j < per && first + j < a.N;
+      const bool present = first + j < a.N;
       const uint2 v = load_global(present ? reinterpret_cast<const uint2 *>(row + first + j)
                                           : reinterpret_cast<const uint2 *>(&kZeroVector));
       key[j] = normal(v.x);
       key[j + 1] = normal(v.y);
     }
-  } else {
-#pragma unroll
-    for (int j = 0; j < kKeys; ++j) {
-      const bool present = j < per && first + j < a.N;
-      const float *source =
-          present ? row + first + j : reinterpret_cast<const float *>(&kZeroVector);
-      key[j] = normal(__float_as_uint(load_global(source)));
-    }
   }
-  auto valid = [&](int j) { return j < per && first + j < a.N; };
+  auto valid = [&](int j) { return first + j < a.N; };
   // a padded token's scores are all +0, every key one bin's: its first `want`
   // candidates are the ties kept, without the passes (whose LDS atomics would
   // all meet on that bin: select 22.2 us for 16 tokens, 3 of them padded,
@@ -2120,33 +2113,28 @@ __device__ __forceinline__ void select_token(const SelectArgs &a, int t, bool wr
     }
   }
   // the run's selected flags (and completed flags: cleared, or the selected
-  // ones) as one store per 4 or 2 candidates where the run allows
+  // ones) as one store per 4 or 2 candidates (the buffers' own alignment is 1)
   {
+    typedef uint32_t flags4 __attribute__((aligned(1)));
+    typedef uint16_t flags2 __attribute__((aligned(1)));
     uint8_t *selected = a.selected + static_cast<long>(t) * a.N + first;
     uint8_t *completed = a.completed + static_cast<long>(t) * a.N + first;
     auto flag = [&](int j) { return (kept_bits >> j) & 1u; };
-    if (per % 4 == 0) {
+    if constexpr (per % 4 == 0) {
 #pragma unroll
       for (int j = 0; j < kKeys; j += 4)
-        if (j < per && first + j < a.N) {
+        if (first + j < a.N) {
           const uint32_t flags = flag(j) | flag(j + 1) << 8 | flag(j + 2) << 16 | flag(j + 3) << 24;
-          *reinterpret_cast<uint32_t *>(selected + j) = flags;
-          *reinterpret_cast<uint32_t *>(completed + j) = completed_kept ? flags : 0u;
-        }
-    } else if (per % 2 == 0) {
-#pragma unroll
-      for (int j = 0; j < kKeys; j += 2)
-        if (j < per && first + j < a.N) {
-          const uint16_t flags = static_cast<uint16_t>(flag(j) | flag(j + 1) << 8);
-          *reinterpret_cast<uint16_t *>(selected + j) = flags;
-          *reinterpret_cast<uint16_t *>(completed + j) = completed_kept ? flags : 0;
+          *reinterpret_cast<flags4 *>(selected + j) = flags;
+          *reinterpret_cast<flags4 *>(completed + j) = completed_kept ? flags : 0u;
         }
     } else {
 #pragma unroll
-      for (int j = 0; j < kKeys; ++j)
-        if (j < per && first + j < a.N) {
-          selected[j] = static_cast<uint8_t>(flag(j));
-          completed[j] = completed_kept ? static_cast<uint8_t>(flag(j)) : 0;
+      for (int j = 0; j < kKeys; j += 2)
+        if (first + j < a.N) {
+          const uint16_t flags = static_cast<uint16_t>(flag(j) | flag(j + 1) << 8);
+          *reinterpret_cast<flags2 *>(selected + j) = flags;
+          *reinterpret_cast<flags2 *>(completed + j) = completed_kept ? flags : 0;
         }
     }
   }
@@ -3056,7 +3044,7 @@ __global__ __launch_bounds__(kSelectThreads) void select_exact_kernel(SelectArgs
   kept_bits[tid] = kept;
   __syncthreads();
   if (wave >= item_waves) return;
-  const int per = (s.N + kSelectThreads - 1) / kSelectThreads;
+  constexpr int per = kKeys;
   const int q = (static_cast<int>(blockIdx.x) - 1) * item_waves + wave;
   if (q < a.F) {
     // the thread j whose kept run holds position q: lane l reads the end of
@@ -3821,6 +3809,21 @@ static SmallScreenArgs small_screen_args(const Shape &s, const cfmoe_dims *dims,
   return ss;
 }
 
+// Keys per select thread for N candidates: the fewest of these that hold them.
+// The run is a compile-time constant, so no pass tests for keys past it (with
+// 8 or 16 keys and the run at run time, 6144 candidates took 10.4 us at one
+// token, select and exact together, and select 41 us at 1000 tokens; 6 keys
+// take 9.2 and 31.7).
+template <class Launch>
+static void for_select_keys(int n, Launch launch) {
+  const int keys = (n + kSelectThreads - 1) / kSelectThreads;
+  if (keys <= 4) launch(std::integral_constant<int, 4>());
+  else if (keys <= 6) launch(std::integral_constant<int, 6>());
+  else if (keys <= 8) launch(std::integral_constant<int, 8>());
+  else if (keys <= 12) launch(std::integral_constant<int, 12>());
+  else launch(std::integral_constant<int, kSelectKeys>());
+}
+
 static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weights *weights,
                       const cfmoe_workspace *workspace, const void *hidden,
                       const void *router_ids, const void *router_weights,
@@ -3976,9 +3979,10 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
       auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(tokens), dim3(kSelectThreads), 0, stream, sel);
       };
-      const bool few = s.N <= 8 * kSelectThreads;
-      if (sel.read_work) launch(few ? select_kernel<8, true> : select_kernel<kSelectKeys, true>);
-      else launch(few ? select_kernel<8, false> : select_kernel<kSelectKeys, false>);
+      for_select_keys(s.N, [&](auto keys) {
+        constexpr int kKeys = decltype(keys)::value;
+        launch(sel.read_work ? select_kernel<kKeys, true> : select_kernel<kKeys, false>);
+      });
       if ((rc = check_launch("select"))) return rc;
     }
   } else if (stages & (1u << CFMOE_STAGE_SELECT)) {
@@ -4103,13 +4107,11 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
       auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(kSelectThreads), 0, stream, sel, ex, item_waves);
       };
-      const bool few = s.N <= 8 * kSelectThreads;
-      if (sel.read_work)
-        launch(few ? select_exact_kernel<8, kNarrowParts, true>
-                   : select_exact_kernel<kSelectKeys, kNarrowParts, true>);
-      else
-        launch(few ? select_exact_kernel<8, kNarrowParts, false>
-                   : select_exact_kernel<kSelectKeys, kNarrowParts, false>);
+      for_select_keys(s.N, [&](auto keys) {
+        constexpr int kKeys = decltype(keys)::value;
+        launch(sel.read_work ? select_exact_kernel<kKeys, kNarrowParts, true>
+                             : select_exact_kernel<kKeys, kNarrowParts, false>);
+      });
     } else if (hidden_parts(s.H) == kNarrowParts)
       hipLaunchKernelGGL(exact_kernel<kNarrowParts>, dim3(s.F + (encode_items + 1) / 2, tokens), dim3(kWave), 0,
                          stream, ex);
