@@ -24,6 +24,7 @@ IDS_INT64 = 32
 WEIGHTS_BF16 = 64
 INPUT_PREPARED = 128
 CHARGE_KEPT = 256
+ENCODER_TILES = 512
 
 EINVAL = 1
 EHIP = 2

@@ -75,8 +75,8 @@ SelectionScore = Literal["recovery-aware", "point"]
 DOWN_TILE = 32
 REFERENCE_DOWN_TILE = 128
 ENCODER_TILE = 64
-# Recovery rank whose encoder runs inside the exact launch (tile-major coefficients).
-DIRECT_RANK = 32
+# Recovery ranks whose encoder runs inside the exact launch (tile-major coefficients).
+DIRECT_RANKS = (16, 32, 64)
 
 
 def aligned_pairs(pairs: int, experts: int) -> int:
@@ -525,16 +525,16 @@ class ProgressiveReader:
                 encoder.to(device=device, dtype=torch.bfloat16).transpose(1, 2).contiguous()
             )
             self.decoder = decoder.to(device=device, dtype=torch.bfloat16).contiguous()
-            if self.encoder.shape[2] == DIRECT_RANK:
+            if rank in DIRECT_RANKS:
                 # the exact launch's encoder reads each rank's 64 coefficients of
                 # a 64-channel tile as one contiguous row: [E, tiles, R, 64]
                 tiles = ceil(i / ENCODER_TILE)
                 padded = torch.zeros(
-                    (e, tiles * ENCODER_TILE, DIRECT_RANK), dtype=torch.bfloat16, device=device
+                    (e, tiles * ENCODER_TILE, rank), dtype=torch.bfloat16, device=device
                 )
                 padded[:, :i] = self.encoder
                 self._encoder_tiles = (
-                    padded.view(e, tiles, ENCODER_TILE, DIRECT_RANK).transpose(2, 3).contiguous()
+                    padded.view(e, tiles, ENCODER_TILE, rank).transpose(2, 3).contiguous()
                 )
             if selection_score != "point":
                 prepared = True
@@ -724,6 +724,8 @@ class ProgressiveReader:
         if self.selection_threshold is not None:
             flags |= _ext.THRESHOLD | _ext.CHARGE_KEPT
         flags |= _ext.ACCOUNT
+        if self._encoder_tiles is not None:
+            flags |= _ext.ENCODER_TILES
         if ids.dtype == torch.int64:
             flags |= _ext.IDS_INT64
         if weights.dtype == torch.bfloat16:
@@ -1050,10 +1052,11 @@ class ProgressiveReader:
             "grouped_issued_matrix_macs": grouped_macs,
             "workspace_bytes": float(self.workspace_bytes),
             # Below the grouped size an exact workgroup is one wave per kept
-            # channel with no LDS; at rank 32 the encoder workgroups of the
-            # same launch stage two items' 64 channel values (512 B).
+            # channel with no LDS; the encoder workgroups of the same launch
+            # stage 64 / R items' 64 channel values (and, off rank 32, masks).
             "batch_one_completion_shared_bytes_per_cta_upper_bound": float(
-                512 * (self.rank == DIRECT_RANK)
+                64 // self.rank * 64 * (4 if self.rank == 32 else 6)
+                if self.rank in DIRECT_RANKS else 0
             ),
             # No arrival counters (kernel boundaries order the stages), and the
             # selection's radix histograms live in LDS: these global-scratch

@@ -17,7 +17,7 @@
 //   group_exact_kernel  grouped batches: gate/up rows of the channels some
 //                    pair of an expert tile kept, read once per tile (:2655-2718)
 //   encode_kernel    recovery encoder over skipped channels       (:1859-2016)
-//                    (at rank 32 it runs inside the exact launches)
+//                    (at ranks 16, 32 and 64 it runs inside the exact launches)
 //   down_kernel      down rows of kept channels, 32-channel tiles (:1778-1856)
 //   output_kernel    latent, decoder correction, router mix       (:2019-2111)
 //
@@ -2198,7 +2198,7 @@ __global__ void select_all_kernel(SelectArgs a) {
 
 struct EncodeArgs {
   const uint16_t *encoder_t;
-  const uint16_t *encoder_tiles;  // [E, tiles, R, 64] (R = kDirectRank) or NULL
+  const uint16_t *encoder_tiles;  // [E, tiles, R, 64] (direct_rank(R)) or NULL
   const float *partial;
   const uint16_t *activations;
   const uint8_t *completed;
@@ -2277,18 +2277,22 @@ __global__ __launch_bounds__(64) void encode_kernel(EncodeArgs a) {
   encode_tile(a, blockIdx.x, blockIdx.y, blockIdx.z, true, coefficients, kEncodeStride);
 }
 
-// Two (64-channel tile, slot, token) items on one wave at R = kDirectRank:
-// item q = tile + tiles (k + K t) of the flat item order, the wave's pair
-// 2 p and 2 p + 1 (the second may be past `items`: its half stores nothing).
-// Lane 32 h + r takes rank r of item 2 p + h and runs its whole chain over
-// the tile's 64 channels in order. Lanes 32 h + j and 32 h + 32 + j first
-// form item h's values of channels j and 32 + j (zero for a kept channel, a
-// channel past I or a slot with no local expert: fma(0, b, acc) == acc
-// exactly for finite b, since the chain starts at +0 and never holds -0, so
-// a zero value leaves the chain as skipping it would) and put them in LDS,
-// from where every step reads four values of its half's item at once
-// (broadcast reads). The coefficients E[c][r] arrive packed two to a word.
-// Same order and roundings as encode_tile.
+// 64 / R (64-channel tile, slot, token) items on one wave at R = 16, 32 or 64
+// (direct_rank): item q = tile + tiles (k + K t) of the flat item order, the
+// wave's items p 64 / R + h (some may be past `items`: their lanes store
+// nothing). Lane R h + r takes rank r of item h and runs its whole chain over
+// the tile's 64 channels in order. Item h's lanes first form its channels'
+// values (zero for a kept channel, a channel past I or a slot with no local
+// expert: fma(0, b, acc) == acc exactly for finite b, since the chain starts
+// at +0 and never holds -0, so a zero value leaves the chain as skipping it
+// would) and put them in LDS, from where every step reads four values of its
+// item at once (broadcast reads). The coefficients E[c][r] arrive packed two
+// to a word; at R = 16 and 64 those of channels without a value are masked to
+// zero, so that there even an infinite coefficient leaves the chain alone.
+// Same order and roundings as encode_tile. Run inside the exact launches, the
+// items cost less than a launch of encode_kernel (Qwen3 at 256 Zipf tokens,
+// rank 64: exact 182 and encode 38 us apart, 198 together; at 31 tokens, rank
+// 16: 33.6 and 7.8, together 34.3).
 //
 // The selected and completed flags come from the workspace (one-wave
 // workgroups, whose LDS values array is the function's own), or, in a
@@ -2297,6 +2301,9 @@ __global__ __launch_bounds__(64) void encode_kernel(EncodeArgs a) {
 // completed flag (a skipped channel is never completed), the values through
 // the wave's own LDS rows `staged`.
 constexpr int kDirectRank = 32;
+__host__ __device__ inline bool direct_rank(int rank) { return rank == 16 || rank == kDirectRank || rank == 64; }
+// waves of `items` encoder items at a direct rank
+__host__ __device__ inline int encode_blocks(int items, int rank) { return (items * rank + 63) / 64; }
 
 struct WorkspaceFlags {};
 struct KeptBits {
@@ -2304,32 +2311,40 @@ struct KeptBits {
   int per;
 };
 
-template <class Args, class Flags = WorkspaceFlags>  // Args: EncodeArgs or the grouped exact launch's
-__device__ __forceinline__ void encode_pair_direct(const Args &a, int p, int items, int t_base,
-                                                   Flags flags = Flags(), float (*staged)[64] = nullptr) {
-  constexpr int R = kDirectRank;
+// A wave's LDS: its items' values, then (R = 16, 64) its coefficient masks.
+template <int R>
+struct EncodeStage {
+  alignas(16) float values[64 / R][64];
+  alignas(16) uint16_t masks[R == kDirectRank ? 1 : 64 / R][R == kDirectRank ? 1 : 64];
+};
+
+template <int R, class Args, class Flags = WorkspaceFlags>  // Args: EncodeArgs or the grouped exact launch's
+__device__ __forceinline__ void encode_direct(const Args &a, int p, int items, int t_base,
+                                              Flags flags = Flags(), EncodeStage<R> *staged = nullptr) {
   constexpr bool kFromBits = std::is_same<Flags, KeptBits>::value;
-  __shared__ __align__(16) float own_values[kFromBits ? 1 : 2][64];
-  float (*channel_values)[64] = kFromBits ? staged : own_values;
+  constexpr bool kMasked = R != kDirectRank;
+  constexpr int kItems = 64 / R, kOwn = 64 / R;  // items per wave, channels per lane
+  __shared__ EncodeStage<R> own_stage;  // (unused, so not allocated, with KeptBits)
+  EncodeStage<R> &stage = kFromBits ? *staged : own_stage;
   const int lane = threadIdx.x & 63;
-  const int h = lane >> 5, r = lane & 31;
-  const int q = min(2 * p + h, items - 1);
-  const bool store = 2 * p + h < items;
+  const int h = lane / R, r = lane % R;
+  const int q = min(kItems * p + h, items - 1);
+  const bool store = kItems * p + h < items;
   const int tile = q % a.tiles, rest = q / a.tiles;
   const int k = rest % a.K, t = t_base + rest / a.K;
-  // the item's expert (lanes of a half agree); the flag and value loads
+  // the item's expert (an item's lanes agree); the flag and value loads
   // below do not wait for it
   const int e = load_global(a.ids + t * a.K + k);
   const bool active = is_active(a.padding, t);
-  // the item's flags and values of channels r and 32 + r
+  // the item's flags and values of channels r, R + r, ...
   const long flat = static_cast<long>(t) * a.N + static_cast<long>(k) * a.I + tile * 64;
   const long base = static_cast<long>(t) * 2 * a.N + static_cast<long>(k) * a.I + tile * 64;
-  uint8_t is_selected[2], is_completed[2];
-  uint16_t exact[2];
-  float gate[2], up[2];
+  uint8_t is_selected[kOwn], is_completed[kOwn];
+  uint16_t exact[kOwn];
+  float gate[kOwn], up[kOwn];
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const int j = 32 * s + r;
+  for (int s = 0; s < kOwn; ++s) {
+    const int j = R * s + r;
     const bool inside = tile * 64 + j < a.I;
     const long at = inside ? j : 0;
     if constexpr (kFromBits) {
@@ -2361,12 +2376,13 @@ __device__ __forceinline__ void encode_pair_direct(const Args &a, int p, int ite
     coefficient[4 * m + 3] = w.w;
   }
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
+  for (int s = 0; s < kOwn; ++s) {
     const bool skip = local && !is_selected[s];
     float value = 0.0f;
     if (skip)
       value = is_completed[s] ? bf16f(exact[s]) : bfr(cfm_activate(bfr(gate[s]), a.gelu != 0) * bfr(up[s]));
-    channel_values[h][32 * s + r] = value;
+    stage.values[h][R * s + r] = value;
+    if constexpr (kMasked) stage.masks[h][R * s + r] = skip ? 0xffffu : 0u;
   }
   if constexpr (kFromBits) {
     // the wave's own rows: its LDS writes before its reads (in order within
@@ -2377,11 +2393,16 @@ __device__ __forceinline__ void encode_pair_direct(const Args &a, int p, int ite
   } else {
     __syncthreads();  // one-wave workgroups: orders the LDS writes before the reads
   }
-  const float4 *values = reinterpret_cast<const float4 *>(channel_values[h]);
+  const float4 *values = reinterpret_cast<const float4 *>(stage.values[h]);
   float acc = 0.0f;
 #pragma unroll
   for (int g = 0; g < 16; ++g) {
     const float4 v = values[g];
+    if constexpr (kMasked) {
+      const uint2 m = reinterpret_cast<const uint2 *>(stage.masks[h])[g];
+      coefficient[2 * g] &= m.x;
+      coefficient[2 * g + 1] &= m.y;
+    }
     acc = fmaf(v.x, __uint_as_float(coefficient[2 * g] << 16), acc);
     acc = fmaf(v.y, __uint_as_float(coefficient[2 * g] & 0xffff0000u), acc);
     acc = fmaf(v.z, __uint_as_float(coefficient[2 * g + 1] << 16), acc);
@@ -2419,7 +2440,7 @@ struct GroupExactArgs {
   uint8_t *completed;
   int H, I, K, N, F, T, gelu, channel_groups, tile_items;
   int dense;  // every channel kept by every pair (no tile masks)
-  // recovery encoder items (R = kDirectRank) run past the exact tiles
+  // recovery encoder items (direct_rank(R)) run past the exact tiles
   const uint16_t *encoder_t;
   const uint16_t *encoder_tiles;
   float *parts;  // encoder partials
@@ -2603,6 +2624,7 @@ constexpr int kExactChannels = 2;  // channels of one tile per grouped exact wav
 // results of a padded token or of slots with no local expert, and the rest
 // (the grid's tile items past the tile count) have nothing to do. Returns
 // the tile item index of a work workgroup, or -1 when its part is done.
+template <int R>
 __device__ __forceinline__ int group_exact_side_items(const GroupExactArgs &a, int threads) {
   int block = blockIdx.x;
   if (a.down_order) {
@@ -2625,14 +2647,14 @@ __device__ __forceinline__ int group_exact_side_items(const GroupExactArgs &a, i
   const int live_items = min(load_uniform(a.group_total) * a.channel_groups, a.tile_items);
   if (block < live_items) return block;
   const int item = block - live_items;
-  const int encode_blocks = (a.encode_items + 1) / 2;
-  if (item < encode_blocks) {
-    // two recovery encoder items (tile, slot, token), tile fastest; they read
-    // no exact result (a skipped channel is never completed)
-    encode_pair_direct(a, item, a.encode_items, 0);
+  const int encoders = encode_blocks(a.encode_items, R);
+  if (item < encoders) {
+    // a wave's recovery encoder items (tile, slot, token), tile fastest; they
+    // read no exact result (a skipped channel is never completed)
+    encode_direct<R>(a, item, a.encode_items, 0);
     return -1;
   }
-  const int t = item - encode_blocks;
+  const int t = item - encoders;
   if (t >= a.T) return -1;  // (and the tile items past the tile count)
   const bool active = is_active(a.padding, t);
   for (int k = 0; k < a.K; ++k) {
@@ -2646,11 +2668,11 @@ __device__ __forceinline__ int group_exact_side_items(const GroupExactArgs &a, i
   return -1;
 }
 
-template <int kParts>
+template <int kParts, int R>
 __global__ __launch_bounds__(64 * kGroupExactWaves) __attribute__((amdgpu_waves_per_eu(kParts == kNarrowParts ? 7 : 4))) void
 group_exact_kernel(GroupExactArgs a) {
   const int lane = threadIdx.x & 63;
-  const int block = group_exact_side_items(a, 64 * kGroupExactWaves);
+  const int block = group_exact_side_items<R>(a, 64 * kGroupExactWaves);
   if (block < 0) return;
   const int z = block / a.channel_groups;
   const int c0 = (block % a.channel_groups) * kExactChannels;
@@ -2927,7 +2949,7 @@ struct ExactArgs {
   uint16_t *activations;
   uint8_t *completed;
   int H, I, K, N, F, gelu;
-  // recovery encoder items (R = kDirectRank) of the token, one per workgroup
+  // recovery encoder items (direct_rank(R)) of the token, 64 / R per workgroup
   // past exact_blocks (0: none); encode reads no exact result (a skipped
   // channel is never completed)
   EncodeArgs encode;
@@ -2989,13 +3011,13 @@ __device__ __forceinline__ void exact_channel(const ExactArgs &a, int t, int log
 // hidden rows with every part in flight (buffer resources: parts past H, and
 // a padded token's hidden row, read zeros); the chain is row_dots, as in
 // group_exact_kernel.
-template <int kParts>
+template <int kParts, int R>
 __global__ __launch_bounds__(64) void exact_kernel(ExactArgs a) {
   const int lane = threadIdx.x;
   const int t = blockIdx.y;
   if (static_cast<int>(blockIdx.x) >= a.exact_blocks) {
-    const int item = blockIdx.x - a.exact_blocks;  // (tile, slot), tile fastest
-    if (2 * item < a.encode_items) encode_pair_direct(a.encode, item, a.encode_items, t);
+    // the wave's items (tile, slot), tile fastest
+    encode_direct<R>(a.encode, blockIdx.x - a.exact_blocks, a.encode_items, t);
     return;
   }
   const int f = blockIdx.x;
@@ -3024,12 +3046,12 @@ __global__ __launch_bounds__(64) void exact_kernel(ExactArgs a) {
 // before the selection. The host sizes item_waves so that the workgroups
 // (one per compute unit at 16 waves of this kernel's registers) run in one
 // round: the rows then come through as many compute units as that allows.
-template <int kKeys, int kParts, bool kCharge>
+template <int kKeys, int kParts, bool kCharge, int R>
 __global__ __launch_bounds__(kSelectThreads) void select_exact_kernel(SelectArgs s, ExactArgs a,
                                                                       int item_waves) {
   __shared__ int kept_end[kSelectThreads];
   __shared__ uint32_t kept_bits[kSelectThreads];
-  __shared__ __align__(16) float values[kSelectWaves][2][64];
+  __shared__ EncodeStage<R> stages[kSelectWaves];
   const int t = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool writer = blockIdx.x == 0;
@@ -3060,8 +3082,8 @@ __global__ __launch_bounds__(kSelectThreads) void select_exact_kernel(SelectArgs
     for (int n = q - before; n > 0; --n) bits &= bits - 1;
     const int logical = __builtin_amdgcn_readfirstlane(j * per + __builtin_ctz(bits));
     exact_channel<kParts>(a, t, logical, slot_id, padded);
-  } else if (2 * (q - a.F) < a.encode_items) {
-    encode_pair_direct(a.encode, q - a.F, a.encode_items, t, KeptBits{kept_bits, per}, values[wave]);
+  } else if ((q - a.F) * (64 / R) < a.encode_items) {
+    encode_direct<R>(a.encode, q - a.F, a.encode_items, t, KeptBits{kept_bits, per}, &stages[wave]);
   }
 }
 
@@ -3824,6 +3846,15 @@ static void for_select_keys(int n, Launch launch) {
   else launch(std::integral_constant<int, kSelectKeys>());
 }
 
+// The exact launches are compiled for each rank whose encoder items they run
+// (one kernel for all three would hold the widest one's registers).
+template <class Launch>
+static void for_encoder_rank(int rank, bool tiled, Launch launch) {
+  if (tiled && rank == 16) launch(std::integral_constant<int, 16>());
+  else if (tiled && rank == 64) launch(std::integral_constant<int, 64>());
+  else launch(std::integral_constant<int, kDirectRank>());
+}
+
 static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weights *weights,
                       const cfmoe_workspace *workspace, const void *hidden,
                       const void *router_ids, const void *router_weights,
@@ -3837,8 +3868,9 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   if (tokens * s.K > kMaxPairs) return fail(CFMOE_EINVAL, "tokens * top_k exceeds 8192 pairs");
   if (s.R > 0 && (!weights->encoder_t || !weights->decoder))
     return fail(CFMOE_EINVAL, "rank > 0 needs encoder and decoder");
-  if (s.R == kDirectRank && (!weights->encoder_tiles || reinterpret_cast<uintptr_t>(weights->encoder_tiles) % 16))
-    return fail(CFMOE_EINVAL, "encoder_tiles (16-byte aligned) is required at rank 32");
+  const bool tiled = s.R == kDirectRank || (direct_rank(s.R) && (dims->flags & CFMOE_ENCODER_TILES));
+  if (tiled && (!weights->encoder_tiles || reinterpret_cast<uintptr_t>(weights->encoder_tiles) % 16))
+    return fail(CFMOE_EINVAL, "encoder_tiles (16-byte aligned) is required at rank 32 and with CFMOE_ENCODER_TILES");
   if ((dims->flags & CFMOE_THRESHOLD) && !weights->threshold)
     return fail(CFMOE_EINVAL, "threshold flag without threshold");
   if (s.screened && (!weights->trit_planes || reinterpret_cast<uintptr_t>(weights->trit_planes) % 8))
@@ -3899,7 +3931,7 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   // and exact as one launch (select_exact_kernel, in the exact launch's place)
   // when its workgroups at 16 item waves each fit on the compute units at
   // once (a second round would cost more than the launch saves)
-  const int fused_items = s.F + (s.R == kDirectRank ? (s.encoder_tiles * s.K + 1) / 2 : 0);
+  const int fused_items = s.F + (tiled ? encode_blocks(s.encoder_tiles * s.K, s.R) : 0);
   const bool fuse_select = s.screened && !grouped && tokens <= kSelectExactTokens &&
                            (stages & (1u << CFMOE_STAGE_SELECT)) && (stages & (1u << CFMOE_STAGE_EXACT)) &&
                            hidden_parts(s.H) == kNarrowParts &&
@@ -4009,12 +4041,11 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   en.R = s.R;
   en.tiles = s.encoder_tiles;
   en.gelu = gelu;
-  // At R = kDirectRank the encoder runs inside the exact launch (it needs no
-  // LDS there), which the exact stage launches (also alone, through
+  // With a tile-major encoder the encoder runs inside the exact launch, which the exact stage launches (also alone, through
   // cfmoe_launch_stage); the encode stage then has no launch of its own.
   // Grouped batches build the down kernel's workgroup order (expert-grouped
   // per XCD) in the exact launch and read it in the down launch.
-  const bool encode_in_exact = s.R == kDirectRank;
+  const bool encode_in_exact = tiled;
   const bool fuse_encode = encode_in_exact && (stages & (1u << CFMOE_STAGE_EXACT));
   const int encode_items = fuse_encode ? s.encoder_tiles * s.K : 0;  // per token
   const int down_blocks = (tokens * s.max_tiles + 7) / 8 * 8;
@@ -4066,14 +4097,16 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
     gx.read_work = masked && (flags & CFMOE_ACCOUNT) ? workspace->read_work : nullptr;
     gx.union_row_bytes = 4.0 * s.H;
     const int counters = gx.read_work ? kUnionCounters : 0;
-    if (hidden_parts(s.H) == kNarrowParts)
-      hipLaunchKernelGGL(group_exact_kernel<kNarrowParts>,
-                       dim3(kDownBuilders + counters + gx.tile_items + (gx.encode_items + 1) / 2 + tokens),
-                       dim3(64 * kGroupExactWaves), 0, stream, gx);
-    else
-      hipLaunchKernelGGL(group_exact_kernel<kWideParts>,
-                       dim3(kDownBuilders + counters + gx.tile_items + (gx.encode_items + 1) / 2 + tokens),
-                       dim3(64 * kGroupExactWaves), 0, stream, gx);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel,
+                         dim3(kDownBuilders + counters + gx.tile_items + encode_blocks(gx.encode_items, s.R) + tokens),
+                         dim3(64 * kGroupExactWaves), 0, stream, gx);
+    };
+    for_encoder_rank(s.R, tiled, [&](auto rank) {
+      constexpr int kRank = decltype(rank)::value;
+      launch(hidden_parts(s.H) == kNarrowParts ? group_exact_kernel<kNarrowParts, kRank>
+                                               : group_exact_kernel<kWideParts, kRank>);
+    });
     if ((rc = check_launch("exact"))) return rc;
   } else if (stages & (1u << CFMOE_STAGE_EXACT)) {
     ExactArgs ex;
@@ -4099,7 +4132,7 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
     if (fuse_select) {
       // the fewest item waves per workgroup that fit the launch's workgroups
       // (one per token writing, the rest taking items) on the compute units
-      const int items = s.F + (encode_items + 1) / 2;  // fused_items
+      const int items = s.F + encode_blocks(encode_items, s.R);  // fused_items
       const long groups = std::max(1L, compute_units() / tokens - 1);
       const int item_waves =
           static_cast<int>(std::min<long>(kSelectWaves, std::max<long>(1, (items + groups - 1) / groups)));
@@ -4109,15 +4142,22 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
       };
       for_select_keys(s.N, [&](auto keys) {
         constexpr int kKeys = decltype(keys)::value;
-        launch(sel.read_work ? select_exact_kernel<kKeys, kNarrowParts, true>
-                             : select_exact_kernel<kKeys, kNarrowParts, false>);
+        for_encoder_rank(s.R, tiled, [&](auto rank) {
+          constexpr int kRank = decltype(rank)::value;
+          launch(sel.read_work ? select_exact_kernel<kKeys, kNarrowParts, true, kRank>
+                               : select_exact_kernel<kKeys, kNarrowParts, false, kRank>);
+        });
       });
-    } else if (hidden_parts(s.H) == kNarrowParts)
-      hipLaunchKernelGGL(exact_kernel<kNarrowParts>, dim3(s.F + (encode_items + 1) / 2, tokens), dim3(kWave), 0,
-                         stream, ex);
-    else
-      hipLaunchKernelGGL(exact_kernel<kWideParts>, dim3(s.F + (encode_items + 1) / 2, tokens), dim3(kWave), 0,
-                         stream, ex);
+    } else {
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(s.F + encode_blocks(encode_items, s.R), tokens), dim3(kWave), 0, stream, ex);
+      };
+      for_encoder_rank(s.R, tiled, [&](auto rank) {
+        constexpr int kRank = decltype(rank)::value;
+        launch(hidden_parts(s.H) == kNarrowParts ? exact_kernel<kNarrowParts, kRank>
+                                                 : exact_kernel<kWideParts, kRank>);
+      });
+    }
     if ((rc = check_launch("exact"))) return rc;
   }
 

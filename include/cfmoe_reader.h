@@ -47,6 +47,8 @@ typedef struct ihipStream_t *cfmoe_stream;
 #define CFMOE_IDS_INT64 32u     /* router ids are int64 (else int32) */
 #define CFMOE_WEIGHTS_BF16 64u  /* router weights are bf16 (else fp32) */
 #define CFMOE_INPUT_PREPARED 128u /* cfmoe_prepare_input already rotated */
+#define CFMOE_ENCODER_TILES 512u /* rank 16 or 64: encoder_tiles is given, and the encoder
+                                   runs inside the exact launch (as always at rank 32) */
 #define CFMOE_CHARGE_KEPT 256u  /* with CFMOE_ACCOUNT: also add the read statistics that
                                    follow each token's kept count (slots 0, 3, 6, 7, 12,
                                    13, 19); for thresholded calls, whose `charges` then
@@ -58,11 +60,11 @@ typedef struct ihipStream_t *cfmoe_stream;
 #define CFMOE_STAGE_SCORE 2   /* split sums and channel scores (launches nothing: the
                                  screen launch scores) */
 #define CFMOE_STAGE_SELECT 3  /* per-token top-F */
-#define CFMOE_STAGE_EXACT 4   /* native gate/up rows of kept channels (and at rank 32 the
-                                 encoder) */
-#define CFMOE_STAGE_ENCODE 5  /* recovery encoder over skipped channels; at rank 32 it
-                                 runs inside the exact launch, and this stage launches
-                                 nothing */
+#define CFMOE_STAGE_EXACT 4   /* native gate/up rows of kept channels (and, with a tile-major
+                                 encoder, the encoder) */
+#define CFMOE_STAGE_ENCODE 5  /* recovery encoder over skipped channels; at rank 32 and with
+                                 CFMOE_ENCODER_TILES it runs inside the exact launch, and
+                                 this stage launches nothing */
 #define CFMOE_STAGE_DOWN 6    /* down rows of kept channels */
 #define CFMOE_STAGE_OUTPUT 7  /* latent, decoder correction, router mix */
 #define CFMOE_STAGE_COUNT 8
@@ -101,8 +103,8 @@ typedef struct cfmoe_weights {
   const float *threshold;  /* [1] selection threshold or NULL */
   const uint32_t *trit_planes; /* screen layout of `codes` (cfmoe_pack_trit_planes) */
   const void *encoder_tiles;   /* bf16 [E, ceil(I/64), R, 64]: encoder_t tile-major, channels past
-                                  I zero; required at R == 32 (the exact launch's encoder), else
-                                  unused */
+                                  I zero; required at R == 32 and with CFMOE_ENCODER_TILES (the
+                                  exact launch's encoder), else unused */
 } cfmoe_weights;
 
 /* Caller-allocated scratch, sized for `capacity` tokens (sizes in bytes from

@@ -313,3 +313,37 @@ def test_thresholded_read_statistics_follow_the_selection(tokens, rank, score):
         want[12] = 4 * h * kept
     assert {slot: work[slot] for slot in want} == want
     assert 0 < kept < count * plan.final_count or tokens == 1
+
+
+@pytest.mark.parametrize("tokens", [2, 9, 16, 40])
+@pytest.mark.parametrize("rank,width", [(16, 80), (64, 80), (16, 256), (64, 272), (48, 80)])
+def test_encoder_items_of_every_rank(tokens, rank, width):
+    """The encoder inside the exact launches (ranks 16 and 64: a last tile of
+    16 channels, item counts that leave a wave part empty) against the oracle,
+    and bit for bit against encode_kernel, which a host without the tile-major
+    copy runs; rank 48 always does. An infinite coefficient of a kept channel
+    stays out of the latent."""
+    layer = make_layer(hidden=512, width=width, experts=8, top_k=3, rank=rank, tokens=tokens, seed=140 + rank)
+    plan = compile_budget(hidden_size=512, expert_width=width, top_k=3, retention=0.25, screen_keep=0.625)
+    reader = build(layer, plan, tokens, selection_score="point")
+    out, expected = run_both(reader, layer, plan, layer.hidden, layer.ids, layer.weights)
+    assert_parity(reader, out, expected, tokens)
+    assert (reader._encoder_tiles is not None) == (rank != 48)
+    # a channel every token that routes to its expert keeps
+    kept = torch.ones(8, width, dtype=torch.bool, device=DEVICE)
+    ids = reader.ids[:tokens].long()
+    for t in range(tokens):
+        kept[ids[t]] &= reader.selected[t].view(3, width)
+    touched = torch.zeros(8, dtype=torch.bool, device=DEVICE)
+    touched[ids.flatten()] = True
+    infinite = layer.encoder.clone()
+    infinite.transpose(1, 2)[(kept & touched[:, None]).cpu()] = float("inf")
+    layer.encoder = infinite
+    outs = []
+    for tiled in (True, False):
+        reader = build(layer, plan, tokens, selection_score="point")
+        if not tiled:
+            reader._encoder_tiles = None
+            reader._weights_c.encoder_tiles = None
+        outs.append(reader(layer.hidden.to(DEVICE), layer.ids.to(DEVICE), layer.weights.to(DEVICE)))
+    assert torch.equal(outs[0], out) and torch.equal(outs[1], out)
