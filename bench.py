@@ -159,7 +159,7 @@ STAGE_KERNELS = {"prepare": "prepare_kernel", "screen": "small_screen_kernel",
                  "select": "select_kernel", "exact": "exact_kernel",
                  "encode": "encode_kernel", "down": "down_kernel", "output": "output_kernel"}
 GROUP_EXACT_TOKENS = GROUPED_TOKENS  # batches from which the exact stage runs group_exact_kernel
-WIDE_OUTPUT_TOKENS = 64  # batches from which the output stage runs output_wide_kernel (top-k <= 16)
+STREAM_OUTPUT_TOKENS = 64  # batches from which the output stage runs output_stream_kernel
 
 
 def encoder_in_exact(tokens: int, rank: int) -> bool:
@@ -185,8 +185,8 @@ def stage_kernel(stage: str, tokens: int) -> str:
         return "group_exact_kernel"
     if stage == "screen" and tokens >= _ext.FUSED_SCREEN_TOKENS:
         return "fused_screen_kernel"
-    if stage == "output" and tokens >= WIDE_OUTPUT_TOKENS:
-        return "output_wide_kernel"
+    if stage == "output" and tokens >= STREAM_OUTPUT_TOKENS:
+        return "output_stream_kernel"
     return STAGE_KERNELS[stage]
 
 
@@ -536,7 +536,7 @@ def summarize_trace(directory: str, command: str) -> str:
     """Per-kernel launch statistics of a rocprofv3 --kernel-trace --stats run."""
     durations: dict[str, list[int]] = {}
     reader_kernels = set(STAGE_KERNELS.values()) | {"select_all_kernel", "group_exact_kernel",
-                                                     "fused_screen_kernel", "output_wide_kernel",
+                                                     "fused_screen_kernel", "output_stream_kernel",
                                                      "output_staged_kernel", "select_exact_kernel"}
     for row in _rocprof_rows(directory, "kernel_trace.csv"):
         name = _short_name(row["Kernel_Name"])

@@ -44,7 +44,16 @@ namespace cfmoe {
 constexpr int kWave = 64;
 constexpr int kMaxSlots = 64;  // top_k limit of the C-ABI
 constexpr int kMaxRank = 64;   // recovery rank limit of the C-ABI
-constexpr int kDownTile = 32;  // selected channels per down tile (one fp32 partial each)
+constexpr int kDownTile = 32;  // selected channels per down tile
+
+// FP32 partials the down launch leaves for a slot of `count` kept channels: one
+// sum of its first `prefix` tiles, added in order, and one of each later tile
+// (only a slot's first tiles can be added up before the others, the sum being
+// ((t0 + t1) + t2) + ...).
+__host__ __device__ inline int down_partials(int count, int prefix) {
+  const int tiles = (count + kDownTile - 1) / kDownTile;
+  return tiles < prefix ? (tiles > 0) : tiles - prefix + 1;
+}
 
 // ---------------------------------------------------------------------------
 // scalar helpers (identical formulas in oracle/cfmoe_oracle.c)
@@ -1858,6 +1867,7 @@ struct SelectArgs {
   int32_t *tile_starts;
   int32_t *down_tile_starts;
   int N, F, I, K;
+  int down_prefix;  // down_tile_starts counts down_partials(count, down_prefix)
   int thresholded;
   // read statistics of the kept count (kCharge), or NULL: rows of
   // hidden size H, encoder rows of rank R; `row_charge` is slot 12's bytes per
@@ -2157,7 +2167,7 @@ __device__ __forceinline__ void select_token(const SelectArgs &a, int t, bool wr
     const bool slot = tid < a.K;
     const int start = slot ? slot_start[tid] : 0;
     const int count = slot ? slot_start[tid + 1] - start : 0;
-    const int tiles = (count + 127) / 128, tiles16 = (count + kDownTile - 1) / kDownTile;
+    const int tiles = (count + 127) / 128, tiles16 = down_partials(count, a.down_prefix);
     const int tile = wave_inclusive(tiles) - tiles, tile16 = wave_inclusive(tiles16) - tiles16;
     if (slot) {
       a.counts[t * a.K + tid] = count;
@@ -2188,7 +2198,7 @@ __global__ void select_all_kernel(SelectArgs a) {
       a.counts[t * a.K + k] = a.I;
       a.starts[t * a.K + k] = k * a.I;
       a.tile_starts[t * a.K + k] = k * ((a.I + 127) / 128);
-      a.down_tile_starts[t * a.K + k] = k * ((a.I + kDownTile - 1) / kDownTile);
+      a.down_tile_starts[t * a.K + k] = k * down_partials(a.I, a.down_prefix);
     }
   }
 }
@@ -2451,7 +2461,7 @@ struct GroupExactArgs {
   int32_t *down_order;
   const int32_t *pair_tiles;
   const int32_t *down_tile_starts;
-  int max_tiles, down_blocks, order_words, slot_capacity;
+  int max_tiles, down_blocks, order_words, slot_capacity, down_prefix;
   // union-row accounting (or NULL): kUnionCounters workgroups after the
   // builders add union_row_bytes to slot 12 per nonzero tile mask word
   double *read_work;
@@ -2525,7 +2535,7 @@ __device__ void build_down_order(const GroupExactArgs &a, int x) {
     for (int u = 0; u < 4; ++u) {
       const int i = i0 + kWave * u + lane;
       if (i >= pairs) continue;
-      const int tiles = (count[u] + kDownTile - 1) / kDownTile;
+      const int tiles = down_partials(count[u], a.down_prefix);
       total += tiles;
       if (slot[u] >= 0)
         records[slot[u]] = make_uint2(tiles, static_cast<uint32_t>((i / a.K) * a.max_tiles + first[u]));
@@ -2572,7 +2582,7 @@ __device__ void build_down_order(const GroupExactArgs &a, int x) {
     for (int u = 0; u < 4; ++u) {
       const int i = i0 + kWave * u + lane;
       const bool outside = i < pairs && slot[u] < 0;
-      place(outside ? (count[u] + kDownTile - 1) / kDownTile : 0,
+      place(outside ? down_partials(count[u], a.down_prefix) : 0,
             (min(i, pairs - 1) / a.K) * a.max_tiles + first[u]);
     }
   }
@@ -2800,25 +2810,30 @@ struct DownArgs {
   const int32_t *down_tile_starts;
   const int32_t *order;  // workgroup b's item t * max_tiles + tile (-1: none), or NULL
   float *parts;
-  int H, I, K, N, F, max_tiles;
+  int H, I, K, N, F, max_tiles, prefix;
   const void *padding_source;  // the padding mask and T bytes, or any pointer and 0 bytes
   int padding_bytes;
 };
 
 constexpr int kDownOutputs = 8;  // outputs per down thread (H / 8 threads)
 
-// The slot of a token's down tile: the slot whose tiles hold it, the tile's
-// first position in the slot's kept list, and the slot's count, expert and
-// start in next_ids (k = -1: the tile is past the token's tiles).
+// The slot of a token's partial: the slot whose partials hold it, the first
+// position in the slot's kept list and the position past the last, the slot's
+// expert and start in next_ids (k = -1: past the token's partials).
 struct DownTile {
   int k, first, count, e, start;
 };
+
+__device__ __forceinline__ void down_range(DownTile &d, int at, int count, int prefix) {
+  d.first = at == 0 ? 0 : (prefix + at - 1) * kDownTile;
+  d.count = at == 0 ? min(count, prefix * kDownTile) : min(count, d.first + kDownTile);
+}
 
 // At K = 8 the token's four records arrive through the scalar cache in one
 // round trip.
 __device__ __forceinline__ DownTile down_tile_slot(const int32_t *counts, const int32_t *tile_starts,
                                                    const int32_t *ids, const int32_t *starts,
-                                                   int K, int t, int tile) {
+                                                   int K, int t, int tile, int prefix) {
   DownTile d = {-1, 0, 0, -1, 0};
   if (K == 8) {
     const long row = static_cast<long>(t) * 8;
@@ -2829,10 +2844,9 @@ __device__ __forceinline__ DownTile down_tile_slot(const int32_t *counts, const 
     asm volatile("" ::"s"(c8), "s"(t8), "s"(e8), "s"(s8));
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      if (tile >= t8[s] && tile < t8[s] + (c8[s] + kDownTile - 1) / kDownTile) {
+      if (tile >= t8[s] && tile < t8[s] + down_partials(c8[s], prefix)) {
         d.k = s;
-        d.first = (tile - t8[s]) * kDownTile;
-        d.count = c8[s];
+        down_range(d, tile - t8[s], c8[s], prefix);
         d.e = e8[s];
         d.start = s8[s];
       }
@@ -2841,10 +2855,9 @@ __device__ __forceinline__ DownTile down_tile_slot(const int32_t *counts, const 
     for (int s = 0; s < K; ++s) {
       const int c = counts[t * K + s];
       const int ts = tile_starts[t * K + s];
-      if (tile >= ts && tile < ts + (c + kDownTile - 1) / kDownTile) {
+      if (tile >= ts && tile < ts + down_partials(c, prefix)) {
         d.k = s;
-        d.first = (tile - ts) * kDownTile;
-        d.count = c;
+        down_range(d, tile - ts, c, prefix);
       }
     }
     if (d.k >= 0) {
@@ -2874,65 +2887,74 @@ __global__ __launch_bounds__(512) void down_kernel(DownArgs a) {
     tile = item % a.max_tiles;
     t = item / a.max_tiles;
   }
-  const DownTile d = down_tile_slot(a.counts, a.down_tile_starts, a.ids, a.starts, a.K, t, tile);
-  const int k = d.k, first = d.first, count = d.count, e = d.e, start = d.start;
+  const DownTile d = down_tile_slot(a.counts, a.down_tile_starts, a.ids, a.starts, a.K, t, tile, a.prefix);
+  const int k = d.k, count = d.count, e = d.e, start = d.start;
   if (k < 0 || tile >= a.max_tiles) return;
-  // the tile's channel ids and the token's padding flag in one round trip
-  const int j = first + (lane & (kDownTile - 1));
-  const int logical = load_global(a.next_ids + static_cast<long>(t) * a.F + min(start + j, a.F - 1));
-  const uint32_t padded =
-      __builtin_amdgcn_raw_buffer_load_b8(buffer_resource(a.padding_source, a.padding_bytes), t, 0, 0);
-  asm volatile("" ::"v"(logical), "v"(padded));
-  const bool local = __builtin_amdgcn_readfirstlane(padded) == 0 && e >= 0;
-  const bool valid = j < count && start + j < a.F && logical >= 0 && logical < a.N;
-  // the tile's valid ids: the prefix before the first invalid one
-  const uint32_t invalid = static_cast<uint32_t>(__ballot(!valid));
-  const uint32_t live = invalid ? (1u << __builtin_ctz(invalid)) - 1u : 0xffffffffu;
-  const int channel = valid ? logical % a.I : 0;
   // z: 512-output chunk of the per-token launch's one-wave workgroups (the
   // grouped launch has one chunk)
   const int o = (blockIdx.z * kWave + tid) * kDownOutputs;
   const bool outputs = o < a.H;
-  // the expert's rows through one buffer resource (none without a local
-  // expert: every row then reads zeros), row c at scalar offset 2 H c; rows
-  // past the live prefix read channel 0's row, which the chain never uses
-  const __amdgpu_buffer_rsrc_t rows =
-      buffer_resource(a.down + (local ? static_cast<long>(e) * a.I * a.H : 0), local ? 2 * a.I * a.H : 0);
   const int column = 2 * min(o, a.H - kDownOutputs);
-  uint4 w[kDownTile];
+  float sum[kDownOutputs];
+  // the partial's tiles in order: one, or a slot's first ones (no branch on
+  // `first` inside: the first tile is taken as it is, -0 + x == x)
 #pragma unroll
-  for (int jj = 0; jj < kDownTile; ++jj) {
-    const int c = __builtin_amdgcn_readlane(channel, jj);
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rows, column, 2 * a.H * c, 0);
-    w[jj] = make_uint4(v.x, v.y, v.z, v.w);
-  }
-  const bool mine = (live >> (lane & (kDownTile - 1))) & 1u;
-  const uint16_t act_bits =
-      load_global(mine ? a.activations + static_cast<long>(t) * a.N + logical
-                       : reinterpret_cast<const uint16_t *>(&kZeroVector));
-  // (every row load is issued before the first is used)
-  asm volatile("" ::: "memory");
-  const int act_lane = static_cast<int>(__float_as_uint(bf16f(act_bits)));
-  // (every lane stays active through the chain: its lane reads fetch
-  // activations from lanes whose outputs may lie past H)
-  float acc[kDownOutputs];
+  for (int i = 0; i < kDownOutputs; ++i) sum[i] = -0.0f;
+  for (int first = d.first; first < count; first += kDownTile) {
+    // the tile's channel ids and the token's padding flag in one round trip
+    const int j = first + (lane & (kDownTile - 1));
+    const int logical = load_global(a.next_ids + static_cast<long>(t) * a.F + min(start + j, a.F - 1));
+    const uint32_t padded =
+        __builtin_amdgcn_raw_buffer_load_b8(buffer_resource(a.padding_source, a.padding_bytes), t, 0, 0);
+    asm volatile("" ::"v"(logical), "v"(padded));
+    const bool local = __builtin_amdgcn_readfirstlane(padded) == 0 && e >= 0;
+    const bool valid = j < count && start + j < a.F && logical >= 0 && logical < a.N;
+    // the tile's valid ids: the prefix before the first invalid one
+    const uint32_t invalid = static_cast<uint32_t>(__ballot(!valid));
+    const uint32_t live = invalid ? (1u << __builtin_ctz(invalid)) - 1u : 0xffffffffu;
+    const int channel = valid ? logical % a.I : 0;
+    // the expert's rows through one buffer resource (none without a local
+    // expert: every row then reads zeros), row c at scalar offset 2 H c; rows
+    // past the live prefix read channel 0's row, which the chain never uses
+    const __amdgpu_buffer_rsrc_t rows =
+        buffer_resource(a.down + (local ? static_cast<long>(e) * a.I * a.H : 0), local ? 2 * a.I * a.H : 0);
+    uint4 w[kDownTile];
 #pragma unroll
-  for (int i = 0; i < kDownOutputs; ++i) acc[i] = 0.0f;
-#pragma unroll
-  for (int jj = 0; jj < kDownTile; ++jj) {
-    if (!((live >> jj) & 1u)) break;
-    const float act = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(act_lane, jj)));
-    const uint32_t wv[4] = {w[jj].x, w[jj].y, w[jj].z, w[jj].w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      acc[2 * i] = fmaf(__uint_as_float(wv[i] << 16), act, acc[2 * i]);
-      acc[2 * i + 1] = fmaf(__uint_as_float(wv[i] & 0xffff0000u), act, acc[2 * i + 1]);
+    for (int jj = 0; jj < kDownTile; ++jj) {
+      const int c = __builtin_amdgcn_readlane(channel, jj);
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rows, column, 2 * a.H * c, 0);
+      w[jj] = make_uint4(v.x, v.y, v.z, v.w);
     }
+    const bool mine = (live >> (lane & (kDownTile - 1))) & 1u;
+    const uint16_t act_bits =
+        load_global(mine ? a.activations + static_cast<long>(t) * a.N + logical
+                         : reinterpret_cast<const uint16_t *>(&kZeroVector));
+    // (every row load is issued before the first is used)
+    asm volatile("" ::: "memory");
+    const int act_lane = static_cast<int>(__float_as_uint(bf16f(act_bits)));
+    // (every lane stays active through the chain: its lane reads fetch
+    // activations from lanes whose outputs may lie past H)
+    float acc[kDownOutputs];
+#pragma unroll
+    for (int i = 0; i < kDownOutputs; ++i) acc[i] = 0.0f;
+#pragma unroll
+    for (int jj = 0; jj < kDownTile; ++jj) {
+      if (!((live >> jj) & 1u)) break;
+      const float act = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(act_lane, jj)));
+      const uint32_t wv[4] = {w[jj].x, w[jj].y, w[jj].z, w[jj].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        acc[2 * i] = fmaf(__uint_as_float(wv[i] << 16), act, acc[2 * i]);
+        acc[2 * i + 1] = fmaf(__uint_as_float(wv[i] & 0xffff0000u), act, acc[2 * i + 1]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kDownOutputs; ++i) sum[i] = sum[i] + acc[i];
   }
   if (!outputs) return;
   float *out = a.parts + (static_cast<long>(t) * a.max_tiles + tile) * a.H + o;
-  *reinterpret_cast<float4 *>(out) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-  *reinterpret_cast<float4 *>(out + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+  *reinterpret_cast<float4 *>(out) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+  *reinterpret_cast<float4 *>(out + 4) = make_float4(sum[4], sum[5], sum[6], sum[7]);
 }
 
 // ---------------------------------------------------------------------------
@@ -3104,7 +3126,8 @@ struct OutputArgs {
   float *latent;
   uint16_t *out;
   int H, K, R, max_tiles, encoder_tiles;
-  int columns;  // outputs per workgroup (64 or 256, at most kOutputThreads)
+  int columns;  // outputs per workgroup (at most kOutputThreads)
+  int down_prefix;
 };
 
 constexpr int kOutputThreads = 512;
@@ -3353,124 +3376,141 @@ __global__ __launch_bounds__(kOutputThreads) void output_staged_kernel(OutputArg
   a.out[static_cast<long>(t) * a.H + o] = f2bf(routed + correction);
 }
 
-constexpr int kOutputItems = 8;      // (slot, output) items per thread: K x columns <= 8 x 512
-constexpr int kWideTileBatch = 4;        // tile partials of an item loaded with the other items'
+// The output launch of grouped batches: every wave takes 256 outputs of a token
+// (four per lane) through all of the token's tile partials, which lie slot
+// after slot in tile order: one 16-byte load and four adds per tile and lane,
+// kStreamTiles tiles in flight ahead of those being added. A slot's end is a
+// scalar test; its sum is rounded and mixed into the outputs at once (the slots
+// come in order), so no slot value is staged. The workgroup folds the token's
+// encoder tiles meanwhile. Same sums and roundings as output_kernel.
+//
+// A thread per (slot, output) item with its own tile bounds spent 14 vector
+// instructions per partial (29 M wave instructions at 1000 Qwen3 tokens, two
+// thirds of that launch's 71 us; this one reads the same partials in 62).
+constexpr int kStreamTiles = 8;
+constexpr int kStreamOutputs = 4;  // outputs per lane
 
-// The output launch from 128 tokens (512 outputs per workgroup): the same
-// arithmetic as output_kernel in two round trips, first the token's slot
-// records (into LDS), each thread's encoder tiles and its output's decoder
-// row, then the tile partials of all of the thread's (slot k, output) items
-// at once (c4: 26.7 -> 23.4 us; below 128 tokens, where a workgroup holds
-// fewer items, output_kernel's order is faster). Each
-// item sums its slot's 32-channel tile partials in tile order and rounds to
-// BF16; one thread per output then mixes the slots in order with the router
-// weights and adds the decoder correction. The per-(slot, output) values
-// live in dynamic LDS.
-__global__ __launch_bounds__(kOutputThreads) void output_wide_kernel(OutputArgs a) {
+__global__ __launch_bounds__(kOutputThreads) void output_stream_kernel(OutputArgs a) {
   __shared__ float slot_latent[kMaxSlots * kMaxRank];
   __shared__ __align__(16) float latent[kMaxRank];  // bf16(latent_r) of the token
-  __shared__ float slot_weight[kMaxSlots];
-  __shared__ int slot_first[kMaxSlots], slot_tiles[kMaxSlots];
-  extern __shared__ float slot_value[];  // [K][columns]
-  const int t = blockIdx.y, tid = threadIdx.x;
-  const int columns = a.columns;
-  const int o0 = blockIdx.x * columns;
+  const int t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, threads = blockDim.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int K = a.K, R = a.R;
-  const int o = o0 + tid;
-  const bool mine = tid < columns && o < a.H;
-  // round trip 1: slot records, encoder tiles, decoder row
-  for (int k = tid; k < K; k += kOutputThreads) {
-    slot_weight[k] = a.weights[t * K + k];
-    const int first = a.down_tile_starts[t * K + k];
-    slot_first[k] = first;
-    slot_tiles[k] = min((a.counts[t * K + k] + kDownTile - 1) / kDownTile, a.max_tiles - first);
-  }
-  const bool direct_encoder = K * R <= kOutputThreads && a.encoder_tiles <= kMaxEncoderTiles;
-  float encoder_v[kMaxEncoderTiles];
-  if (direct_encoder && tid < K * R) {
-    const float *parts = a.encoder_parts + (static_cast<long>(t) * K + tid / R) * a.encoder_tiles * R + tid % R;
+  const int o = (blockIdx.x * (threads / kWave) + wave) * (kWave * kStreamOutputs) + kStreamOutputs * lane;
+  // the partials through one resource over the token's tiles (a tile past
+  // them reads zeros), tile g at scalar offset 4 H g
+  const __amdgpu_buffer_rsrc_t parts =
+      buffer_resource(a.down_parts + static_cast<long>(t) * a.max_tiles * a.H, 4 * a.max_tiles * a.H);
+  float4 now[kStreamTiles], next[kStreamTiles];
+  auto load_tiles = [&](int g0, float4 (&v)[kStreamTiles]) {
 #pragma unroll
-    for (int j = 0; j < kMaxEncoderTiles; ++j) encoder_v[j] = j < a.encoder_tiles ? parts[j * R] : 0.0f;
-  }
-  const bool active = is_active(a.padding, t);
-  const bool row_ahead = R > 0 && a.decoder && (R & 7) == 0 && R <= 32;
-  uint4 decoder_row[4];
-  if (row_ahead) {
-    const uint16_t *row = a.decoder + static_cast<long>(min(o, a.H - 1)) * R;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      decoder_row[q] = 8 * q < R && active ? *reinterpret_cast<const uint4 *>(row + 8 * q) : make_uint4(0, 0, 0, 0);
-  }
-  __syncthreads();
-  // round trip 2: the tile partials of the thread's items (the first
-  // kWideTileBatch tiles of each together; longer slots continue in batches)
-  const int items = K * columns;
-  float v[kOutputItems][kWideTileBatch];
-  const float *item_parts[kOutputItems];
-  int item_tiles[kOutputItems];
-#pragma unroll
-  for (int i = 0; i < kOutputItems; ++i) {
-    const int item = tid + i * kOutputThreads;
-    const int k = item < items ? item / columns : 0;
-    const int column = item < items ? item % columns : 0;
-    const int first = slot_first[k];
-    item_tiles[i] = item < items ? slot_tiles[k] : 0;
-    item_parts[i] = a.down_parts + (static_cast<long>(t) * a.max_tiles + first) * a.H + min(o0 + column, a.H - 1);
-#pragma unroll
-    for (int j = 0; j < kWideTileBatch; ++j)
-      v[i][j] = j < item_tiles[i] ? item_parts[i][static_cast<long>(j) * a.H] : 0.0f;
-  }
-#pragma unroll
-  for (int i = 0; i < kOutputItems; ++i) {
-    const int item = tid + i * kOutputThreads;
-    if (item >= items) continue;
-    float total = 0.0f;
-#pragma unroll
-    for (int j = 0; j < kWideTileBatch; ++j)
-      if (j < item_tiles[i]) total = j == 0 ? v[i][j] : total + v[i][j];
-    for (int j0 = kWideTileBatch; j0 < item_tiles[i]; j0 += kWideTileBatch) {
-      float w[kWideTileBatch];
-#pragma unroll
-      for (int j = 0; j < kWideTileBatch; ++j)
-        w[j] = item_parts[i][static_cast<long>(min(j0 + j, item_tiles[i] - 1)) * a.H];
-#pragma unroll
-      for (int j = 0; j < kWideTileBatch; ++j)
-        if (j0 + j < item_tiles[i]) total = total + w[j];
+    for (int i = 0; i < kStreamTiles; ++i) {
+      const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(parts, 4 * o, 4 * a.H * (g0 + i), 0);
+      v[i] = make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
     }
-    slot_value[item] = bfr(total);  // item = k * columns + column
-  }
+  };
+  // lane k < K: slot k's record
+  const int own = min(lane, K - 1);
+  const float lane_weight = load_global(a.weights + t * K + own);
+  const int lane_first = load_global(a.down_tile_starts + t * K + own);
+  const int lane_count = load_global(a.counts + t * K + own);
+  load_tiles(0, now);
   // each slot's encoder tiles summed in tile order, rounded to BF16
-  if (direct_encoder) {
-    if (tid < K * R) {
-      float total = encoder_v[0];
+  for (int item = tid; item < K * R; item += threads) {
+    const float *encoder = a.encoder_parts + (static_cast<long>(t) * K + item / R) * a.encoder_tiles * R + item % R;
+    float total = 0.0f;
+    for (int j0 = 0; j0 < a.encoder_tiles; j0 += kMaxEncoderTiles) {
+      float v[kMaxEncoderTiles];
 #pragma unroll
-      for (int j = 1; j < kMaxEncoderTiles; ++j)
-        if (j < a.encoder_tiles) total = total + encoder_v[j];
-      slot_latent[tid] = bfr(total);  // tid = k * R + r
+      for (int j = 0; j < kMaxEncoderTiles; ++j) v[j] = encoder[min(j0 + j, a.encoder_tiles - 1) * R];
+#pragma unroll
+      for (int j = 0; j < kMaxEncoderTiles; ++j)
+        if (j0 + j < a.encoder_tiles) total = j0 + j == 0 ? v[j] : total + v[j];
     }
-  } else {
-    for (int item = tid; item < K * R; item += kOutputThreads) {
-      const int k = item / R, r = item % R;
-      const float *parts = a.encoder_parts + (static_cast<long>(t) * K + k) * a.encoder_tiles * R + r;
-      float total = parts[0];
-      for (int j = 1; j < a.encoder_tiles; ++j) total = total + parts[j * R];
-      slot_latent[k * R + r] = bfr(total);
-    }
+    slot_latent[item] = bfr(total);  // item = k * R + r
   }
+  // lane k: the tile past slot k's last one
+  const int lane_end =
+      lane_first + min(down_partials(lane_count, a.down_prefix), a.max_tiles - lane_first);
+  const int tiles = __builtin_amdgcn_readlane(lane_end, K - 1);
+  float routed[kStreamOutputs], sum[kStreamOutputs];
+#pragma unroll
+  for (int i = 0; i < kStreamOutputs; ++i) {
+    routed[i] = 0.0f;
+    sum[i] = -0.0f;  // (-0 + x == x: a slot's first tile is taken as it is)
+  }
+  int k = 0, end = __builtin_amdgcn_readlane(lane_end, 0);
+  auto end_slot = [&] {
+    const float weight = __uint_as_float(__builtin_amdgcn_readlane(__float_as_int(lane_weight), k));
+#pragma unroll
+    for (int i = 0; i < kStreamOutputs; ++i) {
+      routed[i] = fmaf(bfr(sum[i]), weight, routed[i]);
+      sum[i] = -0.0f;
+    }
+    ++k;
+    end = __builtin_amdgcn_readlane(lane_end, min(k, K - 1));
+  };
+  auto add_tiles = [&](int g0, const float4 (&v)[kStreamTiles]) {
+#pragma unroll
+    for (int i = 0; i < kStreamTiles; ++i) {
+      if (g0 + i >= tiles) break;
+      while (k < K && g0 + i >= end) end_slot();
+      sum[0] = sum[0] + v[i].x;
+      sum[1] = sum[1] + v[i].y;
+      sum[2] = sum[2] + v[i].z;
+      sum[3] = sum[3] + v[i].w;
+    }
+  };
+  for (int g0 = 0; g0 < tiles; g0 += 2 * kStreamTiles) {
+    if (g0 + kStreamTiles < tiles) load_tiles(g0 + kStreamTiles, next);
+    add_tiles(g0, now);
+    if (g0 + kStreamTiles >= tiles) break;
+    if (g0 + 2 * kStreamTiles < tiles) load_tiles(g0 + 2 * kStreamTiles, now);
+    add_tiles(g0 + kStreamTiles, next);
+  }
+  while (k < K) end_slot();
   __syncthreads();
   if (tid < R) {
     float mixed = 0.0f;
-    for (int k = 0; k < K; ++k) mixed = fmaf(slot_latent[k * R + tid], slot_weight[k], mixed);
+    for (int j = 0; j < K; ++j)
+      mixed = fmaf(slot_latent[j * R + tid], load_uniform(a.weights + t * K + j), mixed);
     latent[tid] = bfr(mixed);
     if (blockIdx.x == 0) a.latent[static_cast<long>(t) * R + tid] = mixed;
   }
   __syncthreads();
-  if (!mine) return;
-  float routed = 0.0f;
-  for (int k = 0; k < K; ++k) routed = fmaf(slot_value[k * columns + tid], slot_weight[k], routed);
-  const float correction =
-      R > 0 && a.decoder ? decoder_correction(a, decoder_row, row_ahead, active, o, latent) : 0.0f;
-  a.out[static_cast<long>(t) * a.H + o] = f2bf(routed + correction);
+  if (o >= a.H) return;
+  float correction[kStreamOutputs] = {};
+  if (R > 0 && a.decoder && is_active(a.padding, t)) {
+    const uint16_t *row = a.decoder + static_cast<long>(o) * R;
+    if ((R & 7) == 0) {
+      for (int q = 0; q < R; q += 8) {
+        const float4 l0 = *reinterpret_cast<const float4 *>(latent + q);
+        const float4 l1 = *reinterpret_cast<const float4 *>(latent + q + 4);
+        const float l[8] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
+#pragma unroll
+        for (int n = 0; n < kStreamOutputs; ++n) {
+          const uint4 w = load_global(reinterpret_cast<const uint4 *>(row + n * R + q));
+          const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            correction[n] = fmaf(__uint_as_float(wv[i] << 16), l[2 * i], correction[n]);
+            correction[n] = fmaf(__uint_as_float(wv[i] & 0xffff0000u), l[2 * i + 1], correction[n]);
+          }
+        }
+      }
+    } else {
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int n = 0; n < kStreamOutputs; ++n)
+          correction[n] = fmaf(bf16f(row[n * R + r]), latent[r], correction[n]);
+    }
+  }
+  uint32_t out[kStreamOutputs];
+#pragma unroll
+  for (int n = 0; n < kStreamOutputs; ++n) out[n] = f2bf(routed[n] + bfr(correction[n]));
+  typedef u32x2 output_quad __attribute__((aligned(2)));  // (the caller's tensor)
+  *reinterpret_cast<output_quad *>(a.out + static_cast<long>(t) * a.H + o) =
+      u32x2{out[0] | out[1] << 16, out[2] | out[3] << 16};
 }
 
 // ---------------------------------------------------------------------------
@@ -3846,6 +3886,18 @@ static void for_select_keys(int n, Launch launch) {
   else launch(std::integral_constant<int, kSelectKeys>());
 }
 
+// Tiles of a slot that the down launch adds up before it stores a partial.
+// From 512 tokens eight: Qwen3 at 1000 tokens writes 8.7 instead of 28 partials
+// a token, down 249 -> 234 us and output 62 -> 45. Below, a wave that walks
+// several tiles ends too late: two tiles at 64 tokens took down from 38.4 to
+// 42.3 us, at 128 from 55.7 to 59.4, four at 256 Zipf tokens from 134 to 144.
+constexpr int kDownPrefix = 8;
+constexpr int kDownPrefixTokens = 512;
+
+static int down_prefix(int tokens, const Shape &s) {
+  return tokens >= kDownPrefixTokens && tokens >= s.grouped_tokens ? kDownPrefix : 1;
+}
+
 // The exact launches are compiled for each rank whose encoder items they run
 // (one kernel for all three would hold the widest one's registers).
 template <class Launch>
@@ -3915,6 +3967,7 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   sel.I = s.I;
   sel.K = s.K;
   sel.thresholded = (flags & CFMOE_THRESHOLD) != 0;
+  sel.down_prefix = down_prefix(tokens, s);
   // per-(tile, channel) pair masks for the grouped exact kernel; that launch
   // counts their nonzero words as the union rows it reads (4 H bytes each)
   const bool grouped = tokens >= s.grouped_tokens;
@@ -4091,6 +4144,7 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
     gx.pair_tiles = workspace->pair_tiles;
     gx.down_tile_starts = workspace->down_tile_starts;
     gx.max_tiles = s.max_tiles;
+    gx.down_prefix = sel.down_prefix;
     gx.down_blocks = down_blocks;
     gx.order_words = static_cast<int>(down_list_words(workspace->capacity, s));
     gx.slot_capacity = static_cast<int>(down_slot_capacity(workspace->capacity, s));
@@ -4184,6 +4238,7 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
     dn.N = s.N;
     dn.F = s.F;
     dn.max_tiles = s.max_tiles;
+    dn.prefix = sel.down_prefix;
     dn.padding_source = padding ? static_cast<const void *>(padding) : static_cast<const void *>(weights->signs);
     dn.padding_bytes = padding ? tokens : 0;
     const int down_threads = ((s.H / kDownOutputs + kWave - 1) / kWave) * kWave;
@@ -4216,12 +4271,12 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   op.K = s.K;
   op.R = s.R;
   op.max_tiles = s.max_tiles;
+  op.down_prefix = sel.down_prefix;
   op.encoder_tiles = s.encoder_tiles;
-  // wider workgroups fold each token's encoder tiles fewer times: 512 outputs
-  // from 64 tokens (c3 at 128 tokens: 18.4 -> 14.6 us; at 100 tokens 13.7 ->
-  // 10.0, the launch's workgroups then fit at two per CU), 256 from the
-  // grouped size, 64 below it; LDS K x columns x 4 <= 16 KB
-  op.columns = !grouped ? 64 : s.K <= 8 && tokens >= 64 ? 512 : s.K <= 16 ? 256 : 64;
+  // 256 outputs per workgroup from the grouped size (its workgroups fold their
+  // token's encoder tiles, so wider ones read them fewer times), 64 below it
+  // for latency; LDS K x columns x 4 <= 16 KB
+  op.columns = grouped && s.K <= 16 ? 256 : 64;
   const unsigned value_lds = static_cast<unsigned>(s.K * op.columns * sizeof(float));
   const long staged = static_cast<long>(s.max_tiles) * op.columns;  // partials per workgroup
   const long rounds = (staged + kOutputThreads - 1) / kOutputThreads;
@@ -4229,13 +4284,19 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   const dim3 grid((s.H + op.columns - 1) / op.columns, tokens);
   const bool stageable = s.H % op.columns == 0 && s.K * s.R <= kOutputThreads &&
                          s.encoder_tiles <= kMaxEncoderTiles && rounds <= kStagedRoundsMax;
-  // the two-round-trip kernel (slot records, encoder tiles and decoder row;
-  // then every item's tile partials at once) from 64 tokens, at 512 columns
-  // or, above top-8, 256 (c2's layer 160.9 -> 159.3 us; at 16 and 32 tokens
-  // it measured 0.4-0.6 us slower than the one-pass kernel)
-  if (tokens >= 64 && op.columns >= 256)
-    hipLaunchKernelGGL(output_wide_kernel, grid, dim3(kOutputThreads), value_lds, stream, op);
-  else if (stageable && rounds <= 4)
+  // the streaming kernel from 64 tokens, and for grouped batches whose partials
+  // the staged kernel cannot hold (OLMoE at 64 tokens 9.3 -> 8.9 us, Qwen3 at
+  // 128 10.7 -> 10.4, at 256 Zipf tokens 42 -> 35; 48 tokens of H = 4096, I =
+  // 1536 14.6 -> 13.6). At 16 to 31 tokens the staged kernel's one round trip
+  // is faster (6.4 against 8.1 us at 16, 6.3 against 6.7 at 31)
+  if (grouped && (tokens >= 64 || !stageable)) {
+    const int quads = (s.H + kWave * kStreamOutputs - 1) / (kWave * kStreamOutputs);  // waves per token
+    // two waves per workgroup while the tokens are few (more compute units), a
+    // token's all from 256 tokens (its encoder tiles folded once)
+    const int waves = std::min({quads, kOutputThreads / kWave, tokens >= 256 ? quads : 2});
+    hipLaunchKernelGGL(output_stream_kernel, dim3((quads + waves - 1) / waves, tokens), dim3(kWave * waves), 0,
+                       stream, op);
+  } else if (stageable && rounds <= 4)
     hipLaunchKernelGGL(output_staged_kernel<4>, grid, dim3(kOutputThreads), staged_lds, stream, op);
   else if (stageable && rounds <= 8)
     hipLaunchKernelGGL(output_staged_kernel<8>, grid, dim3(kOutputThreads), staged_lds, stream, op);

@@ -132,7 +132,8 @@ typedef struct cfmoe_workspace {
   int32_t *starts;            /* [cap, K] */
   int32_t *counts;            /* [cap, K] */
   int32_t *tile_starts;       /* [cap, K] 128-channel tiles */
-  int32_t *down_tile_starts;  /* [cap, K] 32-channel tiles */
+  int32_t *down_tile_starts;  /* [cap, K] first down partial: one per 32-channel tile, but from
+                                 512 tokens a slot's first eight tiles share one */
   float *down_parts;          /* [cap, ceil(F/32) + K - 1, H] */
   float *encoder_parts;       /* [cap, K, ceil(I/64), R] */
   float *latent;              /* [cap, R] */
