@@ -2678,8 +2678,91 @@ __device__ __forceinline__ int group_exact_side_items(const GroupExactArgs &a, i
   return -1;
 }
 
-template <int kParts, int R>
-__global__ __launch_bounds__(64 * kGroupExactWaves) __attribute__((amdgpu_waves_per_eu(kParts == kNarrowParts ? 7 : 4))) void
+// The dots of one kept channel with every pair of `mask`, for channels that
+// many pairs keep: the gate and up rows are unpacked to FP32 once (64
+// registers at H = 2048), a pair's hidden row is on its way while the pair
+// before it is used, and two pairs' four sums share one butterfly: after level
+// m = 1 lane l holds the gate (l even) or the up sum of its own two lanes, after
+// m = 2 lanes 4 i .. 4 i + 3 the four sums of their four, and the later levels
+// add equal lanes -- every sum in the order of wave_sum_lane0. H is a multiple
+// of 512 (no part is cut). `store(pair lane, g, u)` receives each pair's sums.
+constexpr int kManyStep = 512;  // hidden coordinates per part
+
+template <class LoadHidden, class Store>
+__device__ __forceinline__ void many_pair_dots(const uint4 (&gw)[kNarrowParts], const uint4 (&uw)[kNarrowParts],
+                                               int H, uint32_t mask, LoadHidden load_hidden, Store store) {
+  const int lane = threadIdx.x & 63;
+  const bool odd = lane & 1, upper = lane & 2;
+  float grow[kNarrowParts][8], urow[kNarrowParts][8];
+  auto unpack = [](const uint4 &w, float (&v)[8]) {
+    const uint32_t wv[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(wv[i] << 16);
+      v[2 * i + 1] = __uint_as_float(wv[i] & 0xffff0000u);
+    }
+  };
+  uint4 x0[kNarrowParts], x1[kNarrowParts];
+  int p0 = __builtin_ctz(mask);
+  load_hidden(p0, x0);
+#pragma unroll
+  for (int j = 0; j < kNarrowParts; ++j) {
+    unpack(gw[j], grow[j]);
+    unpack(uw[j], urow[j]);
+  }
+  auto dots = [&](const uint4 (&xw)[kNarrowParts], float &g, float &u) {
+    g = u = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kNarrowParts; ++j) {
+      if (kManyStep * j >= H) break;
+      float x[8];
+      unpack(xw[j], x);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        g = fmaf(grow[j][i], x[i], g);
+        u = fmaf(urow[j][i], x[i], u);
+      }
+    }
+  };
+  for (uint32_t rest = mask & (mask - 1);;) {
+    float g0, u0, g1, u1;
+    const bool second = rest != 0u;
+    const int p1 = second ? __builtin_ctz(rest) : p0;
+    if (second) load_hidden(p1, x1);
+    dots(x0, g0, u0);
+    if (!second) {
+      store(p0, wave_sum_lane0(g0), wave_sum_lane0(u0));
+      return;
+    }
+    rest &= rest - 1;
+    const int following = rest ? __builtin_ctz(rest) : p0;
+    if (rest) load_hidden(following, x0);
+    dots(x1, g1, u1);
+    auto dpp = [](float v, auto control) {
+      return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(control)::value, 0xf, 0xf, true));
+    };
+    const std::integral_constant<int, 0xb1> xor1;
+    const std::integral_constant<int, 0x4e> xor2;
+    const std::integral_constant<int, 0x104> down4;  // lane i: lane i + 4 of the row of 16
+    const std::integral_constant<int, 0x108> down8;
+    const float first = (odd ? u0 : g0) + dpp(odd ? g0 : u0, xor1);
+    const float other = (odd ? u1 : g1) + dpp(odd ? g1 : u1, xor1);
+    float sums = (upper ? other : first) + dpp(upper ? first : other, xor2);
+    sums = sums + dpp(sums, down4);  // (lanes 0 .. 3 of a row of 16 from here)
+    sums = sums + dpp(sums, down8);
+    sums = sums + lane_xor<16>(sums);
+    sums = sums + lane_xor<32>(sums);
+    auto sum_of = [&](int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sums), i)); };
+    store(p0, sum_of(0), sum_of(1));
+    store(p1, sum_of(2), sum_of(3));
+    if (!rest) return;
+    p0 = following;
+    rest &= rest - 1;
+  }
+}
+
+template <int kParts, int R, bool kMany = false>
+__global__ __launch_bounds__(64 * kGroupExactWaves) __attribute__((amdgpu_waves_per_eu(kParts == kNarrowParts && !kMany ? 7 : 4))) void
 group_exact_kernel(GroupExactArgs a) {
   const int lane = threadIdx.x & 63;
   const int block = group_exact_side_items<R>(a, 64 * kGroupExactWaves);
@@ -2756,7 +2839,7 @@ group_exact_kernel(GroupExactArgs a) {
       for (int j = 0; j < kParts; ++j) xw[j] = buffer_load16(hidden, offset + 1024 * j);
     };
     // the first keeping pair's hidden row travels with the gate/up rows
-    load_hidden(__builtin_ctz(mask));
+    if constexpr (!kMany) load_hidden(__builtin_ctz(mask));
     // rows read once stream past the caches; rows the expert's other tiles read
     // again stay cached for them
     uint4 gw[kParts], uw[kParts];
@@ -2776,7 +2859,19 @@ group_exact_kernel(GroupExactArgs a) {
     // lane p holds pair p's sums; the results are stored after the loop (a
     // store inside it would delay the next pair's loads, which wait in order)
     float kept_g = 0.0f, kept_u = 0.0f;
-    for (uint32_t rest = mask; rest; rest &= rest - 1) {
+    if constexpr (kMany) {
+      auto load_pair = [&](int pp, uint4 (&x)[kParts]) {
+        const int t = __builtin_amdgcn_readlane(token, pp);
+        const __amdgpu_buffer_rsrc_t hidden = buffer_resource(a.x + static_cast<long>(t) * a.H, row_bytes);
+#pragma unroll
+        for (int j = 0; j < kParts; ++j) x[j] = buffer_load16(hidden, offset + 1024 * j);
+      };
+      many_pair_dots(gw, uw, a.H, mask, load_pair, [&](int pp, float g, float u) {
+        kept_g = lane == pp ? g : kept_g;
+        kept_u = lane == pp ? u : kept_u;
+      });
+    }
+    for (uint32_t rest = kMany ? 0u : mask; rest; rest &= rest - 1) {
       const int pp = __builtin_ctz(rest);
       if (rest != mask) load_hidden(pp);
       float g = 0.0f, uu = 0.0f;
@@ -3886,6 +3981,14 @@ static void for_select_keys(int n, Launch launch) {
   else launch(std::integral_constant<int, kSelectKeys>());
 }
 
+// Average keeping pairs of an expert's channel (tokens K F / (E N)) from which
+// the grouped exact kernel unpacks the rows once and reads hidden rows ahead:
+// at 0.98 OLMoE at 64 tokens 69.3 -> 67.7 us and Qwen3 at 128 103.3 -> 102.4,
+// even at 4 and 7.7 (256 Zipf tokens, 1000 tokens: the L2 bounds those); at 0.25
+// its four waves per SIMD lose to seven (34.4 -> 36.6 at 31 tokens, 22.0 ->
+// 23.6 at 16).
+constexpr double kManyPairs = 0.5;
+
 // Tiles of a slot that the down launch adds up before it stores a partial.
 // From 512 tokens eight: Qwen3 at 1000 tokens writes 8.7 instead of 28 partials
 // a token, down 249 -> 234 us and output 62 -> 45. Below, a wave that walks
@@ -4156,10 +4259,15 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
                          dim3(kDownBuilders + counters + gx.tile_items + encode_blocks(gx.encode_items, s.R) + tokens),
                          dim3(64 * kGroupExactWaves), 0, stream, gx);
     };
+    // many_pair_dots where an expert's channel is kept by kManyPairs or more
+    // pairs on average
+    const bool many_pairs = s.H % kManyStep == 0 && hidden_parts(s.H) == kNarrowParts &&
+                            static_cast<double>(tokens) * s.K * s.F >= kManyPairs * dims->experts * s.N;
     for_encoder_rank(s.R, tiled, [&](auto rank) {
       constexpr int kRank = decltype(rank)::value;
-      launch(hidden_parts(s.H) == kNarrowParts ? group_exact_kernel<kNarrowParts, kRank>
-                                               : group_exact_kernel<kWideParts, kRank>);
+      launch(many_pairs                             ? group_exact_kernel<kNarrowParts, kRank, true>
+             : hidden_parts(s.H) == kNarrowParts ? group_exact_kernel<kNarrowParts, kRank>
+                                                 : group_exact_kernel<kWideParts, kRank>);
     });
     if ((rc = check_launch("exact"))) return rc;
   } else if (stages & (1u << CFMOE_STAGE_EXACT)) {
