@@ -2472,10 +2472,15 @@ constexpr int kMaxHidden = 4096;
 constexpr int kDownBuilders = 8;     // one per XCD
 constexpr int kUnionCounters = 64;  // workgroups counting the tile masks' nonzero words
 // 16-byte parts per lane of a hidden-size row: 4 up to H = 2048 (the common
-// shapes, 72 VGPRs in the grouped kernel), 8 up to kMaxHidden
+// shapes, 72 VGPRs in the grouped kernel), 6 up to 3072 (at H = 2816 eight parts
+// cost more instructions and a wave per SIMD: grouped exact at 24 tokens 37.6 us,
+// six 35.8), 8 up to kMaxHidden
 constexpr int kNarrowParts = 4;
+constexpr int kMiddleParts = 6;
 constexpr int kWideParts = kMaxHidden / 512;
-__host__ __device__ inline int hidden_parts(int H) { return H <= 512 * kNarrowParts ? kNarrowParts : kWideParts; }
+__host__ __device__ inline int hidden_parts(int H) {
+  return H <= 512 * kNarrowParts ? kNarrowParts : H <= 512 * kMiddleParts ? kMiddleParts : kWideParts;
+}
 
 // Lane-ordered gate and up dots with a hidden row, each row held as kParts
 // 16-byte parts per lane (part j of lane l: h = 512 j + 8 l + i, i < 8): the
@@ -2762,7 +2767,7 @@ __device__ __forceinline__ void many_pair_dots(const uint4 (&gw)[kNarrowParts], 
 }
 
 template <int kParts, int R, bool kMany = false>
-__global__ __launch_bounds__(64 * kGroupExactWaves) __attribute__((amdgpu_waves_per_eu(kParts == kNarrowParts && !kMany ? 7 : 4))) void
+__global__ __launch_bounds__(64 * kGroupExactWaves) __attribute__((amdgpu_waves_per_eu(kMany ? 4 : kParts == kNarrowParts ? 7 : kParts == kMiddleParts ? 5 : 4))) void
 group_exact_kernel(GroupExactArgs a) {
   const int lane = threadIdx.x & 63;
   const int block = group_exact_side_items<R>(a, 64 * kGroupExactWaves);
@@ -4086,11 +4091,13 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   // Up to kSelectExactTokens tokens a call that runs both stages runs select
   // and exact as one launch (select_exact_kernel, in the exact launch's place)
   // when its workgroups at 16 item waves each fit on the compute units at
-  // once (a second round would cost more than the launch saves)
+  // once (a second round would cost more than the launch saves). With six
+  // hidden parts (H = 2816) the fused kernel spills a few registers: one token
+  // 38.8 -> 36.7 us a layer, three 48.8 -> 50.7, so there only one token fuses
   const int fused_items = s.F + (tiled ? encode_blocks(s.encoder_tiles * s.K, s.R) : 0);
   const bool fuse_select = s.screened && !grouped && tokens <= kSelectExactTokens &&
                            (stages & (1u << CFMOE_STAGE_SELECT)) && (stages & (1u << CFMOE_STAGE_EXACT)) &&
-                           hidden_parts(s.H) == kNarrowParts &&
+                           (hidden_parts(s.H) == kNarrowParts || (hidden_parts(s.H) == kMiddleParts && tokens == 1)) &&
                            tokens * (1L + (fused_items + kSelectWaves - 1) / kSelectWaves) <= compute_units();
 
   if (s.screened) {
@@ -4267,6 +4274,7 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
       constexpr int kRank = decltype(rank)::value;
       launch(many_pairs                             ? group_exact_kernel<kNarrowParts, kRank, true>
              : hidden_parts(s.H) == kNarrowParts ? group_exact_kernel<kNarrowParts, kRank>
+             : hidden_parts(s.H) == kMiddleParts ? group_exact_kernel<kMiddleParts, kRank>
                                                  : group_exact_kernel<kWideParts, kRank>);
     });
     if ((rc = check_launch("exact"))) return rc;
@@ -4306,8 +4314,12 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
         constexpr int kKeys = decltype(keys)::value;
         for_encoder_rank(s.R, tiled, [&](auto rank) {
           constexpr int kRank = decltype(rank)::value;
-          launch(sel.read_work ? select_exact_kernel<kKeys, kNarrowParts, true, kRank>
-                               : select_exact_kernel<kKeys, kNarrowParts, false, kRank>);
+          if (hidden_parts(s.H) == kNarrowParts)
+            launch(sel.read_work ? select_exact_kernel<kKeys, kNarrowParts, true, kRank>
+                                 : select_exact_kernel<kKeys, kNarrowParts, false, kRank>);
+          else
+            launch(sel.read_work ? select_exact_kernel<kKeys, kMiddleParts, true, kRank>
+                                 : select_exact_kernel<kKeys, kMiddleParts, false, kRank>);
         });
       });
     } else {
@@ -4316,8 +4328,9 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
       };
       for_encoder_rank(s.R, tiled, [&](auto rank) {
         constexpr int kRank = decltype(rank)::value;
-        launch(hidden_parts(s.H) == kNarrowParts ? exact_kernel<kNarrowParts, kRank>
-                                                 : exact_kernel<kWideParts, kRank>);
+        launch(hidden_parts(s.H) == kNarrowParts   ? exact_kernel<kNarrowParts, kRank>
+               : hidden_parts(s.H) == kMiddleParts ? exact_kernel<kMiddleParts, kRank>
+                                                   : exact_kernel<kWideParts, kRank>);
       });
     }
     if ((rc = check_launch("exact"))) return rc;

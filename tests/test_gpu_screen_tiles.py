@@ -20,9 +20,12 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("score", ["point", "recovery-aware"])
 @pytest.mark.parametrize("hidden,tokens", [
-    (128, 4), (384, 13), (1152, 5), (2048, 4), (2048, 12), (2048, 17), (2176, 5), (2688, 13), (3968, 12),
+    (128, 4), (384, 13), (1152, 5), (2048, 4), (2048, 12), (2048, 17), (2176, 5), (2688, 13), (3072, 1),
+    (3072, 3), (3072, 16), (3200, 1), (3968, 12),
 ])
 def test_screen_tile_edges_bit_exact(hidden, tokens, score):
+    # (the hidden sizes also cover the exact rows' part counts: 4 up to 2048, 6 up
+    # to 3072, 8 above)
     layer = make_layer(hidden=hidden, width=80, experts=2, top_k=2, rank=16, tokens=tokens,
                        seed=300 + hidden + tokens)
     plan = compile_budget(hidden_size=hidden, expert_width=80, top_k=2, retention=0.25, screen_keep=0.625)
