@@ -20,6 +20,8 @@
 //                    (at ranks 16, 32 and 64 it runs inside the exact launches)
 //   down_kernel      down rows of kept channels, 32-channel tiles (:1778-1856)
 //   output_kernel    latent, decoder correction, router mix       (:2019-2111)
+//                    (output_staged_kernel and output_stream_kernel do the
+//                    same where their layouts fit)
 //
 // Arithmetic contract (shared with the CPU oracle, oracle/cfmoe_oracle.c):
 // the screen's per-block dot products are exact integer sums of trits times
@@ -989,10 +991,10 @@ __global__ __launch_bounds__(kPrepareThreads) void prepare_kernel(PrepareArgs a)
 constexpr int kRowTile = 16;
 constexpr int kPairTile = 16;
 static_assert(kPairTile == kGroupPairs, "a screen workgroup holds one grouping tile");
-// Rotation blocks per split: the screens are compiled for a span of 2
+// Rotation blocks per split: the small screen is compiled for a span of 2
 // (H <= 2048: the common shapes, registers and LDS sized for them) and of
 // kMaxSpan (H <= 4096, e.g. Gemma's 2816 = 22 blocks: seven splits of three
-// blocks and one of one).
+// blocks and one of one). The fused screen stages blocks in twos at any span.
 constexpr int kNarrowSpan = 2;
 constexpr int kMaxSpan = 4;
 constexpr int kDigitStride = 144;  // bytes per pair row of a digit plane (128 + pad)
@@ -1270,7 +1272,7 @@ struct SmallScreenArgs {
   float *variances;
   float *scores;
   int H, I, K, N, T, splits, span, tile_items, max_pairs;
-  int gelu, point;
+  int gelu;
 };
 
 // One (block, row tile) step's loads: operand words, FP16 scale (and
@@ -1278,12 +1280,6 @@ struct SmallScreenArgs {
 struct StepLoads {
   uint2 words, scale, residual;
 };
-
-// An empty use of a step's registers: the wait for its loads happens here,
-// on every path, and not where the compiler would merge paths (a loop head).
-__device__ __forceinline__ void consume(const StepLoads &l) {
-  asm volatile("" ::"v"(l.words.x), "v"(l.words.y), "v"(l.scale.x), "v"(l.scale.y));
-}
 
 
 constexpr int kWaveSplits = (kMaxSplits + kSmallWaves - 1) / kSmallWaves;
@@ -1524,7 +1520,7 @@ struct FusedScreenArgs {
   float *scores;
   uint32_t *tile_masks;  // cleared for the wave's channels (or NULL)
   int H, I, K, N, T, splits, span, channel_groups, tile_items;
-  int gelu, point;
+  int gelu;
 };
 
 // Rotation blocks staged together, whatever a split's blocks.
@@ -3999,7 +3995,6 @@ static SmallScreenArgs small_screen_args(const Shape &s, const cfmoe_dims *dims,
   // a tile holds at most 16 pairs, and at most tokens * K
   ss.max_pairs = static_cast<int>(std::min<long>(kPairTile, static_cast<long>(tokens) * s.K));
   ss.gelu = (flags & CFMOE_GELU) != 0;
-  ss.point = (flags & CFMOE_POINT) != 0;
   return ss;
 }
 
@@ -4173,7 +4168,6 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
       fs.channel_groups = (s.I / kRowTile + kFusedWaves - 1) / kFusedWaves;
       fs.tile_items = static_cast<int>(tiles) * fs.channel_groups;
       fs.gelu = gelu;
-      fs.point = !gh5;
       const unsigned blocks = static_cast<unsigned>(fs.tile_items + tokens);
       auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kFusedThreads), 0, stream, fs);
