@@ -3525,15 +3525,18 @@ __global__ __launch_bounds__(kOutputThreads) void output_stream_kernel(OutputArg
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int K = a.K, R = a.R;
   const int o = (blockIdx.x * (threads / kWave) + wave) * (kWave * kStreamOutputs) + kStreamOutputs * lane;
-  // the partials through one resource over the token's tiles (a tile past
-  // them reads zeros), tile g at scalar offset 4 H g
+  // the partials through one resource over the token's tiles, tile g at scalar
+  // offset 4 H g, which the resource's range check need not cover: tiles past
+  // the last and outputs past H repeat the last ones (never used)
   const __amdgpu_buffer_rsrc_t parts =
       buffer_resource(a.down_parts + static_cast<long>(t) * a.max_tiles * a.H, 4 * a.max_tiles * a.H);
+  const int column = 4 * min(o, a.H - kStreamOutputs);
   float4 now[kStreamTiles], next[kStreamTiles];
   auto load_tiles = [&](int g0, float4 (&v)[kStreamTiles]) {
 #pragma unroll
     for (int i = 0; i < kStreamTiles; ++i) {
-      const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(parts, 4 * o, 4 * a.H * (g0 + i), 0);
+      const int g = min(g0 + i, a.max_tiles - 1);
+      const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(parts, column, 4 * a.H * g, 0);
       v[i] = make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
     }
   };
