@@ -18,9 +18,12 @@ padding), a width that is not a multiple of five, and unrotated blocks.
 import pytest
 import torch
 
+from calibration_free_moe.reader import _ext
 from calibration_free_moe.reader.sketch import (
+    ZERO_CODE,
     block_hadamard_signs,
     build_sketch,
+    code_offsets,
     rotate_blocks,
     unpack_sketch,
 )
@@ -112,3 +115,66 @@ def test_device_sketch_tiles_and_offsets(experts, width, hidden, offset):
     clean = ~differ.any(-1)
     torch.testing.assert_close(got_stats.cpu().float()[clean], want_stats.float()[clean],
                                rtol=1e-3, atol=1e-4)
+
+
+@pytest.mark.parametrize(
+    "experts,width,hidden,rotated",
+    # runs of 16 bytes (four blocks to a workgroup: fewer, four, five, and a
+    # workgroup that is short of blocks), 32, 64 and more than a tile; odd block
+    # counts, whose last tail rows have no second block, with and without a body
+    [(2, 3, 128, True), (3, 5, 384, False), (2, 16, 640, True), (1, 40, 512, True), (2, 33, 1152, True),
+     (2, 41, 384, True), (1, 80, 256, False), (2, 160, 128, True), (1, 176, 384, True)],
+)
+def test_device_sketch_writes_every_byte_and_no_other(experts, width, hidden, rotated):
+    """The C entry on buffers that hold 0xff, between guard bytes: every code
+    byte is written (121 where no channel's trits lie), every statistic, and
+    nothing on either side."""
+    generator = torch.Generator().manual_seed(7 * width + hidden)
+    weights = (torch.randn(experts, 2 * width, hidden, generator=generator) * 0.02).bfloat16()
+    signs = block_hadamard_signs(hidden, "cpu") if rotated else None
+    want_codes, want_stats = build_sketch(weights, signs)
+    guard, statistics = 256, 2 * want_stats.numel()
+    codes = torch.full((2 * guard + want_codes.numel(),), 0xFF, dtype=torch.uint8, device=DEVICE)
+    stats = torch.full((2 * guard + statistics,), 0xFF, dtype=torch.uint8, device=DEVICE)
+    rows = weights.to(DEVICE)
+    device_signs = None if signs is None else signs.to(DEVICE)
+    _ext.check(_ext.library().cfmoe_build_sketch(
+        experts, width, hidden, rows.data_ptr(), None if signs is None else device_signs.data_ptr(),
+        codes.data_ptr() + guard, stats.data_ptr() + guard, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    for buffer in (codes, stats):
+        assert bool((buffer[:guard] == 0xFF).all()) and bool((buffer[-guard:] == 0xFF).all())
+    got = codes[guard:-guard].cpu().view(experts, -1)
+    padding = torch.ones(got.shape[1], dtype=torch.bool)
+    padding[code_offsets(2 * width, hidden).flatten()] = False
+    assert bool((got[:, padding] == ZERO_CODE).all())
+    differ = unpack_sketch(got, 2 * width, hidden) != unpack_sketch(want_codes, 2 * width, hidden)
+    assert int(differ.sum()) <= max(2, differ.numel() // 10000)  # (near the threshold)
+    assert int((got != want_codes).sum()) <= int(differ.sum())
+    # 0xffff is a NaN: no statistic is one
+    got_stats = stats[guard:-guard].cpu().view(torch.float16).view(experts, hidden // 128, 2, 2 * width)
+    clean = ~differ.reshape(experts, 2 * width, hidden // 128, 128).any(-1)
+    torch.testing.assert_close(got_stats.permute(0, 3, 1, 2).float()[clean], want_stats.float()[clean],
+                               rtol=1e-3, atol=1e-4)
+
+
+def test_narrow_sketch_does_not_pay_for_a_wide_tile():
+    """A width of 16 fills 8 of a workgroup's 64 code columns: it takes less time
+    than the 160 channels that fill them all (half of it; as long when every
+    workgroup walks 64 columns)."""
+    signs = block_hadamard_signs(2048, DEVICE)
+
+    def fastest(width):
+        weights = torch.randn(128, 2 * width, 2048, device=DEVICE).mul_(0.02).bfloat16()
+        times = []
+        for _ in range(8):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(20):
+                build_sketch(weights, signs, device_kernel=True)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+
+    assert fastest(16) < 0.75 * fastest(160)
