@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "cfmoe_reader.h"
@@ -319,14 +320,23 @@ CFMOE_API int cfmoe_build_sketch(int32_t experts, int32_t width, int32_t hidden,
   const int columns = narrow ? kNarrowColumns : kTileUnits, pack = kTileUnits / columns;
   a.tiles = (a.stride + columns - 1) / columns;
   a.packs = (a.blocks + pack - 1) / pack;
-  const long items = static_cast<long>(experts) * a.tiles * a.packs;
-  if (items > 0x7fffffffL) return fail(CFMOE_EINVAL, "sketch has too many blocks for one launch");
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(items)), dim3(kTileThreads), 0, stream, a);
-  };
-  if (narrow) launch(a.signs ? build_sketch_kernel<true, kNarrowColumns> : build_sketch_kernel<false, kNarrowColumns>);
-  else launch(a.signs ? build_sketch_kernel<true, kTileUnits> : build_sketch_kernel<false, kTileUnits>);
-  return check_launch("build_sketch");
+  // (a launch holds fewer than 2^32 threads: more experts than that take several)
+  const long per_expert = static_cast<long>(a.tiles) * a.packs;
+  const long most = 0xffffffffL / kTileThreads / per_expert;
+  if (most < 1) return fail(CFMOE_EINVAL, "sketch has too many blocks for one launch");
+  for (long first = 0; first < experts; first += most) {
+    const unsigned items = static_cast<unsigned>(std::min<long>(most, experts - first) * per_expert);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(items), dim3(kTileThreads), 0, stream, a);
+    };
+    if (narrow) launch(a.signs ? build_sketch_kernel<true, kNarrowColumns> : build_sketch_kernel<false, kNarrowColumns>);
+    else launch(a.signs ? build_sketch_kernel<true, kTileUnits> : build_sketch_kernel<false, kTileUnits>);
+    if (int rc = check_launch("build_sketch")) return rc;
+    a.weights += most * a.rows * a.hidden;
+    a.codes += most * a.storage;
+    a.stats += most * a.blocks * 2 * a.rows;
+  }
+  return 0;
 }
 
 }  // extern "C"

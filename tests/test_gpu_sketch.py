@@ -178,3 +178,16 @@ def test_narrow_sketch_does_not_pay_for_a_wide_tile():
         return min(times)
 
     assert fastest(16) < 0.75 * fastest(160)
+
+
+def test_device_sketch_of_more_experts_than_a_launch_holds():
+    """8 388 608 workgroups of 512 threads are 2^32, one more than a launch can
+    hold: the experts past them come from a second one."""
+    pattern = (torch.randn(97, 2, 128, generator=torch.Generator().manual_seed(5)) * 0.02).bfloat16().to(DEVICE)
+    want_codes, want_stats = build_sketch(pattern, device_kernel=True)
+    repeats = (1 << 23) // 97 + 1
+    codes, stats = build_sketch(pattern.repeat(repeats, 1, 1), device_kernel=True)
+    for begin in range(0, repeats, 1 << 13):
+        part = codes.view(repeats, 97, -1)[begin : begin + (1 << 13)]
+        assert bool((part == want_codes).all())
+    assert torch.equal(stats.reshape(repeats, 97, -1), want_stats.reshape(1, 97, -1).expand(repeats, -1, -1))
