@@ -3263,8 +3263,8 @@ constexpr int kMaxEncoderTiles = 16; // encoder tiles folded per batch: ceil(I /
 constexpr int kTileBatch = 8;        // tile partials loaded together per thread
 
 // Workgroup = `columns` outputs of one token, 512 threads (64 outputs below
-// 16 tokens for latency, 256 from there: every workgroup folds its token's
-// encoder tiles, so fewer, wider workgroups read them fewer times). Thread
+// 16 tokens for latency and above top-16, else 256: every workgroup folds its
+// token's encoder tiles, so fewer, wider workgroups read them fewer times). Thread
 // item (slot k, output) sums the slot's 32-channel tile partials in tile order
 // (all loads of a batch issued together) and rounds to BF16; one thread per
 // output then mixes the slots in order with the router weights and adds the
@@ -3363,7 +3363,7 @@ __global__ __launch_bounds__(kOutputThreads) void output_kernel(OutputArgs a) {
     const int k = item / columns, column = item % columns;
     const int o = o0 + column;
     const int first = a.down_tile_starts[t * K + k];
-    const int tiles = min((a.counts[t * K + k] + kDownTile - 1) / kDownTile, a.max_tiles - first);
+    const int tiles = min(down_partials(a.counts[t * K + k], a.down_prefix), a.max_tiles - first);
     const float *parts = a.down_parts + (static_cast<long>(t) * a.max_tiles + first) * a.H +
                          min(o, a.H - 1);
     float total = 0.0f;
@@ -4434,12 +4434,20 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   const dim3 grid((s.H + op.columns - 1) / op.columns, tokens);
   const bool stageable = s.H % op.columns == 0 && s.K * s.R <= kOutputThreads &&
                          s.encoder_tiles <= kMaxEncoderTiles && rounds <= kStagedRoundsMax;
-  // the streaming kernel from 64 tokens, and for grouped batches whose partials
-  // the staged kernel cannot hold (OLMoE at 64 tokens 9.3 -> 8.9 us, Qwen3 at
-  // 128 10.7 -> 10.4, at 256 Zipf tokens 42 -> 35; 48 tokens of H = 4096, I =
-  // 1536 14.6 -> 13.6). At 16 to 31 tokens the staged kernel's one round trip
-  // is faster (6.4 against 8.1 us at 16, 6.3 against 6.7 at 31)
-  if (grouped && (tokens >= 64 || !stageable)) {
+  // Below 64 tokens the staged kernel's one round trip is the fastest (6.4 against
+  // 8.1 us at 16, 6.3 against 6.7 at 31); from 64 the streaming kernel (OLMoE at 64
+  // tokens 9.3 -> 8.9 us, Qwen3 at 128 10.7 -> 10.4, at 256 Zipf tokens 42 -> 35).
+  // Partials that the staged kernel cannot hold, below 64 tokens and above top-16
+  // at any size, go to output_kernel while its workgroups run in one round (three
+  // fit a compute unit): a streaming wave walks all of a token's partials, where a
+  // slot's have a thread of their own (budget 0.4 of the channels, 16 tokens: OLMoE
+  // 11.2 against 6.9 us, H = 4096 with I = 1536 19.0 against 13.6, top-24 17.9
+  // against 7.8). Past one round streaming wins again (layers at 0.123: top-24 at
+  // 32 tokens 139 against 140 us, at 63 202 against 209; H = 4096 with I = 1536 at
+  // 56 tokens 397 against 402, at 48 363 against 362).
+  const bool one_round = static_cast<long>(grid.x) * grid.y <= 3 * compute_units();
+  const bool stream_output = stageable ? tokens >= 64 : (tokens >= 64 && s.K <= 16) || !one_round;
+  if (grouped && stream_output) {
     const int quads = (s.H + kWave * kStreamOutputs - 1) / (kWave * kStreamOutputs);  // waves per token
     // two waves per workgroup while the tokens are few (more compute units), a
     // token's all from 256 tokens (its encoder tiles folded once)
