@@ -2937,12 +2937,20 @@ struct DownArgs {
   const int32_t *down_tile_starts;
   const int32_t *order;  // workgroup b's item t * max_tiles + tile (-1: none), or NULL
   float *parts;
-  int H, I, K, N, F, max_tiles, prefix;
+  int H, I, K, N, F, max_tiles;
   const void *padding_source;  // the padding mask and T bytes, or any pointer and 0 bytes
   int padding_bytes;
 };
 
 constexpr int kDownOutputs = 8;  // outputs per down thread (H / 8 threads)
+
+// Tiles of a slot that the down launch adds up before it stores a partial.
+// From 512 tokens eight: Qwen3 at 1000 tokens writes 8.7 instead of 28 partials
+// a token, down 249 -> 234 us and output 62 -> 45. Below, a wave that walks
+// several tiles ends too late: two tiles at 64 tokens took down from 38.4 to
+// 42.3 us, at 128 from 55.7 to 59.4, four at 256 Zipf tokens from 134 to 144.
+constexpr int kDownPrefix = 8;
+constexpr int kDownPrefixTokens = 512;
 
 // The slot of a token's partial: the slot whose partials hold it, the first
 // position in the slot's kept list and the position past the last, the slot's
@@ -2951,16 +2959,25 @@ struct DownTile {
   int k, first, count, e, start;
 };
 
-__device__ __forceinline__ void down_range(DownTile &d, int at, int count, int prefix) {
-  d.first = at == 0 ? 0 : (prefix + at - 1) * kDownTile;
-  d.count = at == 0 ? min(count, prefix * kDownTile) : min(count, d.first + kDownTile);
+// Partials of a slot of `count` kept channels, and the channels of the slot's
+// partial `at` (kPrefix 1: a tile each).
+template <int kPrefix>
+__device__ __forceinline__ int slot_partials(int count) {
+  return kPrefix == 1 ? (count + kDownTile - 1) / kDownTile : down_partials(count, kPrefix);
+}
+
+template <int kPrefix>
+__device__ __forceinline__ void down_range(DownTile &d, int at, int count) {
+  d.first = kPrefix == 1 ? at * kDownTile : at == 0 ? 0 : (kPrefix + at - 1) * kDownTile;
+  d.count = at == 0 ? min(count, kPrefix * kDownTile) : min(count, d.first + kDownTile);
 }
 
 // At K = 8 the token's four records arrive through the scalar cache in one
 // round trip.
+template <int kPrefix>
 __device__ __forceinline__ DownTile down_tile_slot(const int32_t *counts, const int32_t *tile_starts,
                                                    const int32_t *ids, const int32_t *starts,
-                                                   int K, int t, int tile, int prefix) {
+                                                   int K, int t, int tile) {
   DownTile d = {-1, 0, 0, -1, 0};
   if (K == 8) {
     const long row = static_cast<long>(t) * 8;
@@ -2971,9 +2988,9 @@ __device__ __forceinline__ DownTile down_tile_slot(const int32_t *counts, const 
     asm volatile("" ::"s"(c8), "s"(t8), "s"(e8), "s"(s8));
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      if (tile >= t8[s] && tile < t8[s] + down_partials(c8[s], prefix)) {
+      if (tile >= t8[s] && tile < t8[s] + slot_partials<kPrefix>(c8[s])) {
         d.k = s;
-        down_range(d, tile - t8[s], c8[s], prefix);
+        down_range<kPrefix>(d, tile - t8[s], c8[s]);
         d.e = e8[s];
         d.start = s8[s];
       }
@@ -2982,9 +2999,9 @@ __device__ __forceinline__ DownTile down_tile_slot(const int32_t *counts, const 
     for (int s = 0; s < K; ++s) {
       const int c = counts[t * K + s];
       const int ts = tile_starts[t * K + s];
-      if (tile >= ts && tile < ts + down_partials(c, prefix)) {
+      if (tile >= ts && tile < ts + slot_partials<kPrefix>(c)) {
         d.k = s;
-        down_range(d, tile - ts, c, prefix);
+        down_range<kPrefix>(d, tile - ts, c);
       }
     }
     if (d.k >= 0) {
@@ -3003,6 +3020,11 @@ __device__ __forceinline__ DownTile down_tile_slot(const int32_t *counts, const 
 // stops at the count or at the first invalid id, found by a ballot), the ids
 // are broadcast by lane reads and every thread issues the tile's 32 row loads
 // together, then the 32 activations (one per lane, broadcast the same way).
+//
+// kPrefix: tiles of a slot's first partial. Compiled in, since a workgroup counts
+// the partials of every slot it searches: at run time one Qwen3 token took 4.6
+// us, now 4.4, top-24 at 64 tokens 58.6 and now 54.3, top-64 115.6 and 99.9.
+template <int kPrefix>
 __global__ __launch_bounds__(512) void down_kernel(DownArgs a) {
   asm volatile("" ::"s"(a.parts), "s"(a.down), "s"(a.activations), "s"(a.next_ids), "s"(a.padding_source),
                "s"(a.padding_bytes), "s"(a.max_tiles), "s"(a.H), "s"(a.I), "s"(a.N), "s"(a.F));
@@ -3014,7 +3036,7 @@ __global__ __launch_bounds__(512) void down_kernel(DownArgs a) {
     tile = item % a.max_tiles;
     t = item / a.max_tiles;
   }
-  const DownTile d = down_tile_slot(a.counts, a.down_tile_starts, a.ids, a.starts, a.K, t, tile, a.prefix);
+  const DownTile d = down_tile_slot<kPrefix>(a.counts, a.down_tile_starts, a.ids, a.starts, a.K, t, tile);
   const int k = d.k, count = d.count, e = d.e, start = d.start;
   if (k < 0 || tile >= a.max_tiles) return;
   // z: 512-output chunk of the per-token launch's one-wave workgroups (the
@@ -4024,14 +4046,6 @@ static void for_select_keys(int n, Launch launch) {
 // 23.6 at 16).
 constexpr double kManyPairs = 0.5;
 
-// Tiles of a slot that the down launch adds up before it stores a partial.
-// From 512 tokens eight: Qwen3 at 1000 tokens writes 8.7 instead of 28 partials
-// a token, down 249 -> 234 us and output 62 -> 45. Below, a wave that walks
-// several tiles ends too late: two tiles at 64 tokens took down from 38.4 to
-// 42.3 us, at 128 from 55.7 to 59.4, four at 256 Zipf tokens from 134 to 144.
-constexpr int kDownPrefix = 8;
-constexpr int kDownPrefixTokens = 512;
-
 static int down_prefix(int tokens, const Shape &s) {
   return tokens >= kDownPrefixTokens && tokens >= s.grouped_tokens ? kDownPrefix : 1;
 }
@@ -4388,16 +4402,16 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
     dn.N = s.N;
     dn.F = s.F;
     dn.max_tiles = s.max_tiles;
-    dn.prefix = sel.down_prefix;
     dn.padding_source = padding ? static_cast<const void *>(padding) : static_cast<const void *>(weights->signs);
     dn.padding_bytes = padding ? tokens : 0;
     const int down_threads = ((s.H / kDownOutputs + kWave - 1) / kWave) * kWave;
     if (grouped) {
-      hipLaunchKernelGGL(down_kernel, dim3(down_blocks), dim3(down_threads), 0, stream, dn);
+      hipLaunchKernelGGL(sel.down_prefix == 1 ? down_kernel<1> : down_kernel<kDownPrefix>, dim3(down_blocks),
+                         dim3(down_threads), 0, stream, dn);
     } else {
       // one wave per workgroup and 512 outputs each: a batch-1 call's tiles
       // spread over H / 512 times as many CUs
-      hipLaunchKernelGGL(down_kernel, dim3(s.max_tiles, tokens, down_threads / kWave), dim3(kWave),
+      hipLaunchKernelGGL(down_kernel<1>, dim3(s.max_tiles, tokens, down_threads / kWave), dim3(kWave),
                          0, stream, dn);
     }
     if ((rc = check_launch("down"))) return rc;
