@@ -321,8 +321,9 @@ def test_encoder_items_of_every_rank(tokens, rank, width):
     """The encoder inside the exact launches (ranks 16 and 64: a last tile of
     16 channels, item counts that leave a wave part empty) against the oracle,
     and bit for bit against encode_kernel, which a host without the tile-major
-    copy runs; rank 48 always does. An infinite coefficient of a kept channel
-    stays out of the latent."""
+    copy runs; rank 48 always does. An infinite coefficient of a channel that
+    every token of its expert keeps (there need not be one) stays out of the
+    latent."""
     layer = make_layer(hidden=512, width=width, experts=8, top_k=3, rank=rank, tokens=tokens, seed=140 + rank)
     plan = compile_budget(hidden_size=512, expert_width=width, top_k=3, retention=0.25, screen_keep=0.625)
     reader = build(layer, plan, tokens, selection_score="point")
@@ -347,3 +348,35 @@ def test_encoder_items_of_every_rank(tokens, rank, width):
             reader._weights_c.encoder_tiles = None
         outs.append(reader(layer.hidden.to(DEVICE), layer.ids.to(DEVICE), layer.weights.to(DEVICE)))
     assert torch.equal(outs[0], out) and torch.equal(outs[1], out)
+
+
+@pytest.mark.parametrize("tokens", [4, 16, 40])
+@pytest.mark.parametrize("rank,width", [(16, 80), (64, 80), (16, 256), (64, 272)])
+def test_infinite_coefficients_of_kept_channels(tokens, rank, width):
+    """Experts of one or two tokens, so that many channels are kept by every
+    token of theirs, the last, partial tile's among them: infinite encoder
+    coefficients there change no bit, in the exact launches' encoder items below
+    and from the grouped size and in encode_kernel."""
+    layer = make_layer(hidden=512, width=width, experts=64, top_k=3, rank=rank, tokens=tokens, seed=170 + rank)
+    plan = compile_budget(hidden_size=512, expert_width=width, top_k=3, retention=0.25, screen_keep=0.625)
+    arguments = [v.to(DEVICE) for v in (layer.hidden, layer.ids, layer.weights)]
+    reader = build(layer, plan, tokens, selection_score="point")
+    out = reader(*arguments)
+    torch.cuda.synchronize()
+    ids, selected = reader.ids[:tokens].long().cpu(), reader.selected[:tokens].view(tokens, 3, width).cpu()
+    kept = torch.ones(64, width, dtype=torch.bool)
+    for t in range(tokens):
+        kept[ids[t]] &= selected[t]
+    touched = torch.zeros(64, dtype=torch.bool)
+    touched[ids.flatten()] = True
+    kept &= touched[:, None]
+    last = (width - 1) // 64 * 64
+    assert int(kept[:, :last].sum()) > 0 and int(kept[:, last:].sum()) > 0
+    layer.encoder = layer.encoder.clone()
+    layer.encoder.transpose(1, 2)[kept] = float("inf")
+    for tiled in (True, False):
+        reader = build(layer, plan, tokens, selection_score="point")
+        if not tiled:
+            reader._encoder_tiles = None
+            reader._weights_c.encoder_tiles = None
+        assert torch.equal(reader(*arguments), out)
