@@ -34,6 +34,7 @@ import torch  # noqa: E402
 from calibration_free_moe.reader import _ext  # noqa: E402
 from calibration_free_moe.reader.budget import compile_budget  # noqa: E402
 from calibration_free_moe.reader.progressive import (  # noqa: E402
+    DIRECT_RANKS,
     GROUPED_TOKENS,
     ProgressiveReader,
     ReaderWorkspace,
@@ -154,18 +155,18 @@ def algorithmic_bytes(reader: ProgressiveReader, tokens: int) -> dict[str, int]:
 
 STAGE_BYTES = {"screen": ("sketch",), "exact": ("gate_up",), "down": ("down",),
                "encode": ("encoder",)}
-DIRECT_RANK = 32  # rank at which the encoder runs inside the exact launch
 STAGE_KERNELS = {"prepare": "prepare_kernel", "screen": "small_screen_kernel",
                  "select": "select_kernel", "exact": "exact_kernel",
                  "encode": "encode_kernel", "down": "down_kernel", "output": "output_kernel"}
 GROUP_EXACT_TOKENS = GROUPED_TOKENS  # batches from which the exact stage runs group_exact_kernel
-STREAM_OUTPUT_TOKENS = 64  # batches from which the output stage runs output_stream_kernel
+STREAM_OUTPUT_TOKENS = 64  # batches from which the output stage of these layers (top-8, hidden
+                           # size 2048) runs output_stream_kernel
 
 
 def encoder_in_exact(tokens: int, rank: int) -> bool:
     """Whether the exact launch also runs the recovery encoder (the encode
     stage then launches nothing)."""
-    return rank == DIRECT_RANK
+    return rank in DIRECT_RANKS
 
 
 def stage_bytes(stage: str, tokens: int, rank: int) -> tuple[str, ...]:
