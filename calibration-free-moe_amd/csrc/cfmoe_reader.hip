@@ -1492,9 +1492,9 @@ constexpr int kFusedThreads = 64 * kFusedWaves;
 constexpr int kScaleQuads = kRowTile / 4;
 constexpr int kScaleBlock = 2 * kFusedWaves * kScaleQuads;
 // Tokens from which the fused screen runs: the per-channel-tile workgroups of
-// small_screen_kernel do a whole tile's work for each one-pair tile, so from
-// two tokens the fused screen is faster (Qwen3 layer: 13.0 against 17.2 us at
-// 2 tokens, 20.8 against 54.0 at 8; at one token 12.8 against 8.5).
+// small_screen_kernel do a whole tile's work for each one-pair tile: with 2 and 8
+// Qwen3 tokens it took 17.2 and 54.0 us where the fused screen takes 10.5 and
+// 16.7; at one token it takes 6.8, the fused screen took 12.8.
 constexpr int kFusedScreenTokens = 2;
 constexpr int kStageAhead = 1;
 constexpr int kStageBuffers = kStageAhead + 1;
@@ -2793,6 +2793,7 @@ __device__ __forceinline__ void many_pair_dots(const uint4 (&gw)[kNarrowParts], 
   }
 }
 
+// (with four parts at rank 16 one register spills, the price of seven waves)
 template <int kParts, int R, bool kMany = false>
 __global__ __launch_bounds__(64 * kGroupExactWaves) __attribute__((amdgpu_waves_per_eu(kMany ? 4 : kParts == kNarrowParts ? 7 : kParts == kMiddleParts ? 5 : 4))) void
 group_exact_kernel(GroupExactArgs a) {
@@ -2946,9 +2947,11 @@ constexpr int kDownOutputs = 8;  // outputs per down thread (H / 8 threads)
 
 // Tiles of a slot that the down launch adds up before it stores a partial.
 // From 512 tokens eight: Qwen3 at 1000 tokens writes 8.7 instead of 28 partials
-// a token, down 249 -> 234 us and output 62 -> 45. Below, a wave that walks
-// several tiles ends too late: two tiles at 64 tokens took down from 38.4 to
-// 42.3 us, at 128 from 55.7 to 59.4, four at 256 Zipf tokens from 134 to 144.
+// a token, down 247 -> 222 us and output 62 -> 45; at 512 tokens Qwen3's down
+// takes the same 147 us, OLMoE's 171 -> 156, H = 4096 with I = 1536 699 -> 631, and
+// no layer timed from 512 to 1000 was slower. Below, a wave that walks several
+// tiles ends too late: two tiles at 64 tokens took down from 38.4 to 42.3 us, at
+// 128 from 55.7 to 59.4, four at 256 Zipf tokens from 134 to 144.
 constexpr int kDownPrefix = 8;
 constexpr int kDownPrefixTokens = 512;
 
@@ -3284,13 +3287,6 @@ constexpr int kOutputThreads = 512;
 constexpr int kMaxEncoderTiles = 16; // encoder tiles folded per batch: ceil(I / 64) at I <= 1024
 constexpr int kTileBatch = 8;        // tile partials loaded together per thread
 
-// Workgroup = `columns` outputs of one token, 512 threads (64 outputs below
-// 16 tokens for latency and above top-16, else 256: every workgroup folds its
-// token's encoder tiles, so fewer, wider workgroups read them fewer times). Thread
-// item (slot k, output) sums the slot's 32-channel tile partials in tile order
-// (all loads of a batch issued together) and rounds to BF16; one thread per
-// output then mixes the slots in order with the router weights and adds the
-// decoder correction. The per-(slot, output) values live in dynamic LDS.
 // The decoder correction of one output: an fma chain over r of U[o, r] and
 // bf16(latent_r) (`rounded` holds them, 16-byte aligned; a padded token's row
 // is zero), rounded to BF16. `row_words` holds U[o, :] when R is a multiple of
@@ -3349,6 +3345,13 @@ __device__ __forceinline__ void load_decoder_row(const OutputArgs &a, int o0, in
     row_words[q] = 8 * q < a.R ? *reinterpret_cast<const uint4 *>(row + 8 * q) : make_uint4(0, 0, 0, 0);
 }
 
+// Workgroup = `columns` outputs of one token, 512 threads (64 outputs below
+// 16 tokens for latency and above top-16, else 256: every workgroup folds its
+// token's encoder tiles, so fewer, wider workgroups read them fewer times). Thread
+// item (slot k, output) sums the slot's 32-channel tile partials in tile order
+// (all loads of a batch issued together) and rounds to BF16; one thread per
+// output then mixes the slots in order with the router weights and adds the
+// decoder correction. The per-(slot, output) values live in dynamic LDS.
 __global__ __launch_bounds__(kOutputThreads) void output_kernel(OutputArgs a) {
   __shared__ float slot_latent[kMaxSlots * kMaxRank];
   __shared__ __align__(16) float latent[kMaxRank];  // bf16(latent_r) of the token
@@ -3417,15 +3420,15 @@ __global__ __launch_bounds__(kOutputThreads) void output_kernel(OutputArgs a) {
   a.out[static_cast<long>(t) * a.H + o] = f2bf(routed + correction);
 }
 
-// Output below the grouped size in one round trip: every load of the launch
+// Output below 64 tokens in one round trip: every load of the launch
 // is issued before any is used, as buffer loads over the token's ranges (a
 // read past a range returns zero, so none sits behind a branch): the decoder
 // row, the padding flag, the thread's encoder tiles (item tid = k R + r), all
 // max_tiles tile partials of the workgroup's columns (kRounds per thread, into
 // LDS) and the slot records. Each item then sums its slot's tiles from LDS in
-// the order of output_kernel, with the same roundings. The host launches it
-// for K R <= 512 threads, at most kMaxEncoderTiles encoder tiles and
-// max_tiles x columns <= kRounds x 512 partials.
+// the order of output_kernel, with the same roundings (below 64 tokens a slot's
+// partials are its tiles). The host launches it for K R <= 512 threads, at most
+// kMaxEncoderTiles encoder tiles and max_tiles x columns <= kRounds x 512 partials.
 constexpr int kStagedRoundsMax = 16;  // 32 KB of staged partials
 
 template <int kRounds>
@@ -4041,9 +4044,8 @@ static void for_select_keys(int n, Launch launch) {
 // Average keeping pairs of an expert's channel (tokens K F / (E N)) from which
 // the grouped exact kernel unpacks the rows once and reads hidden rows ahead:
 // at 0.98 OLMoE at 64 tokens 69.3 -> 67.7 us and Qwen3 at 128 103.3 -> 102.4,
-// even at 4 and 7.7 (256 Zipf tokens, 1000 tokens: the L2 bounds those); at 0.25
-// its four waves per SIMD lose to seven (34.4 -> 36.6 at 31 tokens, 22.0 ->
-// 23.6 at 16).
+// even at 4 and 7.7 (256 Zipf tokens, 1000 tokens); at 0.25 its four waves per
+// SIMD lose to seven (34.4 -> 36.6 at 31 tokens, 22.0 -> 23.6 at 16).
 constexpr double kManyPairs = 0.5;
 
 static int down_prefix(int tokens, const Shape &s) {
@@ -4136,7 +4138,7 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   // and exact as one launch (select_exact_kernel, in the exact launch's place)
   // when its workgroups at 16 item waves each fit on the compute units at
   // once (a second round would cost more than the launch saves). With six
-  // hidden parts (H = 2816) the fused kernel spills a few registers: one token
+  // hidden parts (H = 2816) the fused kernel spills 12 to 16 registers: one token
   // 38.8 -> 36.7 us a layer, three 48.8 -> 50.7, so there only one token fuses
   const int fused_items = s.F + (tiled ? encode_blocks(s.encoder_tiles * s.K, s.R) : 0);
   const bool fuse_select = s.screened && !grouped && tokens <= kSelectExactTokens &&
