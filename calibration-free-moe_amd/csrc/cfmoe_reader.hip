@@ -4454,14 +4454,17 @@ static int run_stages(uint32_t stages, const cfmoe_dims *dims, const cfmoe_weigh
   // 8.1 us at 16, 6.3 against 6.7 at 31); from 64 the streaming kernel (OLMoE at 64
   // tokens 9.3 -> 8.9 us, Qwen3 at 128 10.7 -> 10.4, at 256 Zipf tokens 42 -> 35).
   // Partials that the staged kernel cannot hold, below 64 tokens and above top-16
-  // at any size, go to output_kernel while its workgroups run in one round (three
-  // fit a compute unit): a streaming wave walks all of a token's partials, where a
-  // slot's have a thread of their own (budget 0.4 of the channels, 16 tokens: OLMoE
-  // 11.2 against 6.9 us, H = 4096 with I = 1536 19.0 against 13.6, top-24 17.9
-  // against 7.8). Past one round streaming wins again (layers at 0.123: top-24 at
-  // 32 tokens 139 against 140 us, at 63 202 against 209; H = 4096 with I = 1536 at
-  // 56 tokens 397 against 402, at 48 363 against 362).
-  const bool one_round = static_cast<long>(grid.x) * grid.y <= 3 * compute_units();
+  // at any size, go to output_kernel while its workgroups run in one round: a
+  // streaming wave walks all of a token's partials, where a slot's have a thread of
+  // their own (budget 0.4 of the channels, 16 tokens: OLMoE 11.2 against 6.9 us, H =
+  // 4096 with I = 1536 19.0 against 13.6, top-24 17.9 against 7.8). Four of its
+  // workgroups fit a compute unit; at 256 columns, four times the work each, a
+  // quarter of the units with a fourth already lose (layers at 0.123, streaming
+  // first: H = 4096 with I = 1536 at 48 tokens, three a unit, 363 and 362 us, at 56
+  // 397 and 401; top-24 at 32 tokens, four a unit, 140 and 139, at 40 157 and 158, at
+  // 63 202 and 209).
+  const int per_unit = op.columns > 64 ? 3 : 4;
+  const bool one_round = static_cast<long>(grid.x) * grid.y <= per_unit * compute_units();
   const bool stream_output = stageable ? tokens >= 64 : (tokens >= 64 && s.K <= 16) || !one_round;
   if (grouped && stream_output) {
     const int quads = (s.H + kWave * kStreamOutputs - 1) / (kWave * kStreamOutputs);  // waves per token

@@ -40,8 +40,9 @@ def test_large_batches_bit_exact(tokens, hidden, width, top_k, rank, retention):
 
 
 @pytest.mark.parametrize("hidden,top_k,rank,tokens", [
-    (2048, 24, 32, 24), (2048, 24, 32, 25), (1024, 33, 16, 48), (1024, 33, 16, 49), (512, 20, 32, 63),
-    (512, 20, 32, 64), (512, 20, 32, 97), (128, 40, 64, 17), (4096, 9, 64, 48), (4096, 9, 64, 49), (4096, 9, 64, 64),
+    (2048, 24, 32, 24), (2048, 24, 32, 32), (2048, 24, 32, 33), (1024, 33, 16, 63), (1024, 33, 16, 64),
+    (1024, 33, 16, 65), (512, 20, 32, 64), (512, 20, 32, 128), (512, 20, 32, 129), (128, 40, 64, 17),
+    (4096, 9, 64, 48), (4096, 9, 64, 49), (4096, 9, 64, 64),
 ])
 def test_unstaged_outputs_bit_exact(hidden, top_k, rank, tokens):
     layer = make_layer(hidden=hidden, width=48, experts=top_k + 2, top_k=top_k, rank=rank, tokens=tokens,
